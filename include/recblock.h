@@ -46,7 +46,11 @@ typedef enum {
 #define RB_SCHED_AUTO 0      /* the library's tuner picks (default) */
 #define RB_SCHED_BLOCKED 1   /* per-block kernels in the reference selector's
                                 order: TRSV, SpMV, TRSV, ... */
-#define RB_SCHED_FUSED 2     /* one persistent dataflow launch per solve */
+#define RB_SCHED_FUSED 2     /* one persistent dataflow launch per solve; for
+                                RB_SCHED_AUTO also the level schedule (one
+                                workgroup per factor and right-hand side),
+                                which the tuner picks for deep, narrow
+                                factors and which has no rb_plan_trace */
 
 typedef struct {
     int schedule;      /* RB_SCHED_* */

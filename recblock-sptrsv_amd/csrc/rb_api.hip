@@ -52,7 +52,7 @@ static int lv_auto(int m, int device_id) {
 // otherwise its first timed solve settles the choice when it is more than
 // twice the fused time (its other two are then not run).
 static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
-    if (p->want_schedule == RB_SCHED_BLOCKED || !p->fused) {
+    if (p->want_schedule == RB_SCHED_BLOCKED || (!p->fused && !p->level)) {
         p->schedule = RB_SCHED_BLOCKED;
         return tune_blocks(p, block_mode, s);
     }
@@ -75,12 +75,14 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     (void)hipEventCreate(&e1);
     // the work of a solve does not depend on the values: b = 0
     if (hipMemsetAsync(db, 0, bytes, s) != hipSuccess) st = RB_ERR_HIP;
+    enum { kBlocked, kFused, kLevel };
     auto timed = [&](int c, int reps) {
         float t = 0.f;
         (void)hipEventRecord(e0, s);
         for (int r = 0; r < reps && st == RB_OK; r++)
-            st = c == 0 ? solve_blocked(p, db, m, dx, m, k, s)
-                        : solve_fused(p, db, m, dx, m, k, s);
+            st = c == kBlocked ? solve_blocked(p, db, m, dx, m, k, s)
+                 : c == kFused ? solve_fused(p, db, m, dx, m, k, s)
+                               : solve_level(p, db, m, dx, m, k, s);
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         (void)hipEventElapsedTime(&t, e0, e1);
@@ -99,31 +101,43 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
         }
         return d != 0;
     };
-    double ms[2] = {0.0, 0.0};
-    bool ok[2] = {true, true}, cut = false;
-    if (st == RB_OK) {
-        (void)timed(1, 1);  // warm
-        ms[1] = timed(1, 3) / 3.0;
-        ok[1] = !tripped();
+    double ms[3] = {0.0, 0.0, 0.0}, best = 0.0;
+    int pick = -1;
+    bool cut = false;
+    for (int c : {kLevel, kFused}) {
+        if (st != RB_OK || (c == kLevel ? !p->level : !p->fused)) continue;
+        (void)timed(c, 1);  // warm
+        ms[c] = timed(c, 3) / 3.0;
+        if (!tripped() && (pick < 0 || ms[c] < best)) {
+            pick = c;
+            best = ms[c];
+        }
     }
+    // The blocked walk goes through every level one after another, at 0.9 us
+    // or more for a level of its fastest kernel, and makes at least four
+    // launches of 4.5 us: not timed where the level schedule takes less than
+    // half of the one or less than the other.
+    const bool clear = pick == kLevel && best < std::max(0.45e-3 * p->nlevel, 0.018);
     if (st == RB_OK)
-        st = tune_blocks(p, block_mode, s, k == 1 && ok[1] ? 2.0 * ms[1] : 0.0,
+        st = tune_blocks(p, clear ? 1 : block_mode, s, k == 1 && pick >= 0 ? 2.0 * best : 0.0,
                          &cut);
-    if (st == RB_OK && !cut) {
-        (void)timed(0, 1);  // warm (captures the walk)
-        const double t1 = timed(0, 1);
-        ms[0] = t1 > 2.0 * ms[1] && ok[1] ? t1 : (t1 + timed(0, 2)) / 3.0;
-        ok[0] = !tripped();
+    if (st == RB_OK && !cut && !clear) {
+        (void)timed(kBlocked, 1);  // warm (captures the walk)
+        const double t1 = timed(kBlocked, 1);
+        ms[kBlocked] = t1 > 2.0 * best && pick >= 0 ? t1 : (t1 + timed(kBlocked, 2)) / 3.0;
+        if (!tripped() && (pick < 0 || ms[kBlocked] <= best)) pick = kBlocked;
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     (void)hipFree(db);
     (void)hipFree(dx);
     if (st != RB_OK) return st;
-    p->tune_ms_blocked = cut ? 0.0 : ms[0];
-    p->tune_ms_fused = ms[1];
-    p->schedule = ok[1] && (cut || !ok[0] || ms[1] < ms[0]) ? RB_SCHED_FUSED
-                                                            : RB_SCHED_BLOCKED;
+    p->tune_ms_blocked = ms[kBlocked];
+    p->tune_ms_fused = pick == kLevel || ms[kFused] == 0.0 ? ms[kLevel] : ms[kFused];
+    p->use_level = pick == kLevel;
+    p->schedule = pick == kLevel || pick == kFused ? RB_SCHED_FUSED : RB_SCHED_BLOCKED;
+    if (p->use_level) fused_destroy(p);
+    else level_destroy(p);
     return RB_OK;
 }
 
@@ -155,6 +169,16 @@ rb_status rb_plan_create(const int *d_colptr, const int *d_rowidx,
                          const double *d_val, int m, int n, int nnz,
                          int substitution, int lv, const rb_opts *opts,
                          void *stream, rb_plan **plan) {
+    return plan_create(d_colptr, d_rowidx, d_val, m, n, nnz, substitution, lv, opts, stream,
+                       nullptr, nullptr, nullptr, 1, plan);
+}
+
+}  // extern "C"
+
+rb_status rb::plan_create(const int *d_colptr, const int *d_rowidx, const double *d_val, int m,
+                          int n, int nnz, int substitution, int lv, const rb_opts *opts,
+                          void *stream, const int *d_part, const int *d_partoff,
+                          const int *h_partoff, int nparts, rb_plan **plan) {
     if (!plan) {
         set_error(RB_ERR_INVALID_ARG, "plan is NULL");
         return RB_ERR_INVALID_ARG;
@@ -190,6 +214,10 @@ rb_status rb_plan_create(const int *d_colptr, const int *d_rowidx,
     p->graph_failed = o.no_graph != 0;  // eager launches only
     p->mixed = o.mixed != 0;
     p->tune_rhs = o.tune_rhs;
+    p->d_part = d_part;
+    p->d_partoff = d_partoff;
+    p->h_partoff = h_partoff;
+    p->nparts = nparts;
     if (o.watchdog_spins > 0) p->spin_limit = (unsigned)o.watchdog_spins;
     rb_status st = RB_OK;
     Arena canon;  // the canonical copy lives until the plan is built
@@ -225,13 +253,17 @@ rb_status rb_plan_create(const int *d_colptr, const int *d_rowidx,
         (void)hipStreamSynchronize((hipStream_t)stream);
         destroy_graph(p);
         fused_destroy(p);
+    level_destroy(p);
         p->arena.release();
         delete p;
         return st;
     }
+    p->h_partoff = nullptr;
     *plan = p;
     return ok();
 }
+
+extern "C" {
 
 rb_status rb_solve(rb_plan *p, const double *d_b, int ldb, double *d_x,
                    int ldx, int nrhs, void *stream) {
@@ -243,7 +275,9 @@ rb_status rb_solve(rb_plan *p, const double *d_b, int ldb, double *d_x,
     if (nrhs == 0) return ok();
     p->mark_first = true;
     rowcap_for_call(p, (hipStream_t)stream);
-    rb_status st = p->schedule == RB_SCHED_FUSED
+    rb_status st = p->use_level
+                       ? solve_level(p, d_b, ldb, d_x, ldx, nrhs, (hipStream_t)stream)
+                   : p->schedule == RB_SCHED_FUSED
                        ? solve_fused(p, d_b, ldb, d_x, ldx, nrhs,
                                      (hipStream_t)stream)
                        : solve_blocked(p, d_b, ldb, d_x, ldx, nrhs,
@@ -340,6 +374,7 @@ rb_status rb_plan_destroy(rb_plan *p) {
     if (p->ev1) (void)hipEventDestroy(p->ev1);
     destroy_graph(p);
     fused_destroy(p);
+    level_destroy(p);
     free_solve_scratch(p);
     p->arena.release();
     delete p;
@@ -374,7 +409,7 @@ rb_status rb_plan_info_get(const rb_plan *p, rb_plan_info *info) {
     info->nlevel = p->nlevel;
     info->schedule = p->schedule;
     info->preprocess_ms = p->preprocess_ms;
-    info->device_bytes = p->arena.bytes;
+    info->device_bytes = p->arena.bytes + level_bytes(p);
     for (int i = 0; i < 4; i++) info->phase_ms[i] = p->phase_ms[i];
     info->tune_ms[0] = p->tune_ms_blocked;
     info->tune_ms[1] = p->tune_ms_fused;

@@ -36,7 +36,12 @@ struct rb_batch {
     // union right-hand sides / solutions, n_total x kalloc column-major
     double *d_B = nullptr, *d_X = nullptr;
     int kalloc = 0;
+    // level schedule: the call's workgroups (pinned, device)
+    int *h_job = nullptr, *d_job = nullptr;
+    size_t job_cap = 0;
     ~rb_batch() {
+        if (h_job) (void)hipHostFree(h_job);
+        if (d_job) (void)hipFree(d_job);
         if (d_B) (void)hipFree(d_B);
         if (d_X) (void)hipFree(d_X);
         if (h_stage) (void)hipHostFree(h_stage);
@@ -192,9 +197,9 @@ rb_status rb_batch_create(int nf, const int *const *d_colptr,
         tmp.release();
         return fail(status_of_hip(hipGetLastError(), "batch assembly"));
     }
-    st = rb_plan_create(ucp, uri, uv, (int)n_total, (int)n_total,
-                        (int)nnz_total, substitution, lv, opts, stream,
-                        &B->plan);
+    st = plan_create(ucp, uri, uv, (int)n_total, (int)n_total, (int)nnz_total,
+                     substitution, lv, opts, stream, B->d_fid, B->d_off, B->off.data(), nf,
+                     &B->plan);
     (void)hipStreamSynchronize(s);
     tmp.release();
     if (st != RB_OK) return fail(st);
@@ -216,12 +221,12 @@ rb_status rb_batch_create(int nf, const int *const *d_colptr,
 
 rb_plan *rb_batch_plan(rb_batch *B) { return B ? B->plan : nullptr; }
 
-// Upload the per-call tables and make sure the union buffers hold kmax
-// columns.  Returns kmax through *kmax.
-static rb_status batch_stage(rb_batch *B, const double *const *d_b,
-                             const int *ldb, double *const *d_x,
-                             const int *ldx, const int *nrhs, hipStream_t s,
-                             int *kmax) {
+// Check the call's arguments and upload its tables, with the level
+// schedule's workgroups when asked for (*njobs of them).
+// Returns the most columns of a factor through *kmax.
+static rb_status batch_tables(rb_batch *B, const double *const *d_b, const int *ldb,
+                              double *const *d_x, const int *ldx, const int *nrhs,
+                              hipStream_t s, int *kmax, int *njobs) {
     const int nf = B->nf;
     int k = 0;
     for (int f = 0; f < nf; f++) {
@@ -235,20 +240,27 @@ static rb_status batch_stage(rb_batch *B, const double *const *d_b,
     }
     *kmax = k;
     if (k == 0 || B->n_total == 0) return RB_OK;
-    if (k > B->kalloc) {
-        RB_HIP(hipStreamSynchronize(s));
-        if (B->d_B) RB_HIP(hipFree(B->d_B));
-        if (B->d_X) RB_HIP(hipFree(B->d_X));
-        B->d_B = B->d_X = nullptr;
-        B->kalloc = 0;
-        const size_t bytes = sizeof(double) * (size_t)B->n_total * k;
-        if (hipMalloc(&B->d_B, bytes) != hipSuccess ||
-            hipMalloc(&B->d_X, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            set_error(RB_ERR_NO_MEMORY, "hipMalloc failed (batch columns)");
-            return RB_ERR_NO_MEMORY;
+    std::vector<int> jobs;
+    if (njobs) {
+        level_jobs(B->plan, nrhs, jobs);
+        *njobs = (int)jobs.size();
+        if (jobs.size() > B->job_cap) {
+            RB_HIP(hipStreamSynchronize(s));
+            RB_HIP(hipEventSynchronize(B->staged));
+            if (B->h_job) RB_HIP(hipHostFree(B->h_job));
+            B->h_job = nullptr;
+            B->job_cap = 0;
+            if (B->d_job) RB_HIP(hipFree(B->d_job));
+            B->d_job = nullptr;
+            const size_t bytes = sizeof(int) * 2 * jobs.size();
+            if (hipHostMalloc(&B->h_job, bytes) != hipSuccess ||
+                hipMalloc(&B->d_job, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                set_error(RB_ERR_NO_MEMORY, "batch workgroup table");
+                return RB_ERR_NO_MEMORY;
+            }
+            B->job_cap = 2 * jobs.size();
         }
-        B->kalloc = k;
     }
     // the previous upload must have been read before the staging buffer
     // is rewritten
@@ -266,7 +278,39 @@ static rb_status batch_stage(rb_batch *B, const double *const *d_b,
                           sizeof(void *) * nf, hipMemcpyHostToDevice, s));
     RB_HIP(hipMemcpyAsync(B->d_ld, hl, sizeof(int) * 3 * nf,
                           hipMemcpyHostToDevice, s));
+    if (!jobs.empty()) {
+        std::memcpy(B->h_job, jobs.data(), sizeof(int) * jobs.size());
+        RB_HIP(hipMemcpyAsync(B->d_job, B->h_job, sizeof(int) * jobs.size(),
+                              hipMemcpyHostToDevice, s));
+    }
     RB_HIP(hipEventRecord(B->staged, s));
+    return RB_OK;
+}
+
+// The tables, and the factors' columns gathered into the union's.
+static rb_status batch_stage(rb_batch *B, const double *const *d_b,
+                             const int *ldb, double *const *d_x,
+                             const int *ldx, const int *nrhs, hipStream_t s,
+                             int *kmax) {
+    const int nf = B->nf;
+    RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, kmax, nullptr));
+    const int k = *kmax;
+    if (k == 0 || B->n_total == 0) return RB_OK;
+    if (k > B->kalloc) {
+        RB_HIP(hipStreamSynchronize(s));
+        if (B->d_B) RB_HIP(hipFree(B->d_B));
+        if (B->d_X) RB_HIP(hipFree(B->d_X));
+        B->d_B = B->d_X = nullptr;
+        B->kalloc = 0;
+        const size_t bytes = sizeof(double) * (size_t)B->n_total * k;
+        if (hipMalloc(&B->d_B, bytes) != hipSuccess ||
+            hipMalloc(&B->d_X, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            set_error(RB_ERR_NO_MEMORY, "hipMalloc failed (batch columns)");
+            return RB_ERR_NO_MEMORY;
+        }
+        B->kalloc = k;
+    }
     const long tot = (long)B->n_total * k;
     k_gather<<<nblk(tot), kT, 0, s>>>(B->d_fid, B->d_off, B->d_bp, B->d_ld, nf,
                                       B->n_total, k, B->d_B);
@@ -296,6 +340,17 @@ rb_status rb_batch_solve(rb_batch *B, const double *const *d_b,
     }
     hipStream_t s = (hipStream_t)stream;
     int k = 0;
+    int widest = 0;
+    for (int f = 0; f < B->nf; f++) widest = std::max(widest, nrhs[f]);
+    if (level_batches(B->plan) && widest <= 0x7fff) {
+        int njobs = 0;
+        RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, &k, &njobs));
+        if (njobs == 0) return done();
+        B->plan->mark_first = true;
+        RB_TRY(solve_level_batch(B->plan, B->d_bp, B->d_xp, B->d_ld, B->d_ld + B->nf,
+                                 B->d_job, njobs, s));
+        return done();
+    }
     RB_TRY(batch_stage(B, d_b, ldb, d_x, ldx, nrhs, s, &k));
     if (k == 0 || B->n_total == 0) return done();
     RB_TRY(rb_solve(B->plan, B->d_B, B->n_total, B->d_X, B->n_total, k, stream));
@@ -318,9 +373,11 @@ rb_status rb_batch_solve_f32ir(rb_batch *B, const double *const *d_b,
     if (relres) *relres = 0.0;
     RB_TRY(batch_stage(B, d_b, ldb, d_x, ldx, nrhs, s, &k));
     if (k == 0 || B->n_total == 0) return done();
+    B->plan->d_partcap = B->d_ld + 2 * B->nf;
     const rb_status st = rb_solve_f32ir(B->plan, B->d_B, B->n_total, B->d_X,
                                         B->n_total, k, tol, max_iter, stream,
                                         iters, relres);
+    B->plan->d_partcap = nullptr;
     if (st != RB_OK && st != RB_ERR_NOT_CONVERGED) return st;
     RB_TRY(batch_unstage(B, k, s));
     if (st != RB_OK) {

@@ -145,6 +145,7 @@ constexpr int kGroupThreads = 1024;
 constexpr int kGroupSlack = 2;   // kTriGroup: rounds a wave may run ahead
 
 struct FusedPlan;
+struct LevelPlan;
 
 }  // namespace rb
 
@@ -199,6 +200,16 @@ struct rb_plan {
     unsigned spin_limit = 1u << 22;  // polls before a bounded wait gives up
     int scratch_rhs = 0;
 
+    // level schedule (rb_level.hip): built for RB_SCHED_AUTO where it
+    // applies; use_level: the tuner picked it
+    rb::LevelPlan *level = nullptr;
+    bool use_level = false;
+    const int *d_part = nullptr;  // independent part of each row (batches)
+    int nparts = 1;
+    const int *d_partoff = nullptr;  // first row of each part
+    const int *h_partoff = nullptr;  // the same on the host (while building)
+    const int *d_partcap = nullptr;  // columns of each part (during a batch call)
+
     // fused schedule (built when requested or for the tuner)
     rb::FusedPlan *fused = nullptr;
     int want_schedule = RB_SCHED_AUTO;
@@ -239,6 +250,12 @@ rb_status canonicalize_csc(const int *d_colptr, const int *d_rowidx,
                            int **c_colptr, int **c_rowidx, double **c_val,
                            int *c_nnz, hipStream_t s);
 
+// rb_plan_create; d_part: the independent part (0 .. nparts - 1) of each row,
+// d_partoff / h_partoff the first row of each (device, host); null for one part
+rb_status plan_create(const int *d_colptr, const int *d_rowidx, const double *d_val, int m,
+                      int n, int nnz, int substitution, int lv, const rb_opts *opts,
+                      void *stream, const int *d_part, const int *d_partoff,
+                      const int *h_partoff, int nparts, rb_plan **plan);
 rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
                      const double *d_val, hipStream_t s);
 rb_status solve_blocked(rb_plan *p, const double *d_b, int ldb, double *d_x,
@@ -271,6 +288,34 @@ rb_status build_fused_finish(FusedJob *job, bool upload);
 rb_status solve_fused(rb_plan *p, const double *d_b, int ldb, double *d_x,
                       int ldx, int nrhs, hipStream_t s);
 void fused_destroy(rb_plan *p);
+// level schedule (rb_level.hip); build_level leaves p->level null when the
+// matrix does not fit it
+rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double *d_cv,
+                      hipStream_t s);
+// from the level widths alone: may the level schedule be the faster one?
+rb_status level_narrow(const rb_plan *p, hipStream_t s, bool *narrow);
+// is the level schedule estimated below the least the fused one takes?
+bool level_beats_chain(const rb_plan *p);
+// ws: per-solve scratch (8 bytes per row and column) instead of the plan's
+rb_status solve_level(rb_plan *p, const double *d_b, int ldb, double *d_x, int ldx,
+                      int nrhs, hipStream_t s, double *ws = nullptr, size_t ws_bytes = 0);
+// one correction of the refinement, as solve_fused32
+rb_status solve_level32(rb_plan *p, const double *d_r, int ldr, double *d_x, int ldx, int nc,
+                        hipStream_t s, const int *left, const int *done);
+// A batch, straight from and to the factors' own columns: one workgroup per
+// (factor, column), listed by level_jobs (column << 16 | factor, or -1 for
+// none; nrhs[f] columns of factor f, at most 0x7fff).
+bool level_batches(const rb_plan *p);
+void level_jobs(const rb_plan *p, const int *nrhs, std::vector<int> &out);
+rb_status solve_level_batch(rb_plan *p, const double *const *d_b, double *const *d_x,
+                            const int *d_ldb, const int *d_ldx, const int *d_job, int njobs,
+                            hipStream_t s);
+// right-hand sides one pass over the columns takes; permuted b / x scratch
+// for ncol of them
+int walk_cols(const rb_plan *p);
+rb_status scratch_cols(rb_plan *p, int ncol, hipStream_t s);
+void level_destroy(rb_plan *p);
+size_t level_bytes(const rb_plan *p);
 // the same solves on caller-provided per-solve buffers (ws, ws_bytes)
 // instead of the plan's: the blocked walk needs blocked_ws_bytes(p) (one
 // column at a time, eager launches), the fused schedule 16 bytes per slot

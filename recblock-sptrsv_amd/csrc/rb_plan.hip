@@ -572,9 +572,13 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     RB_HIP(hipGetLastError());
     RB_TRY(exclusive_scan_i32(prowcnt, prptr, m + 1, s));
 
+    mark("csr");
     // ---- 9, begun here: the fused schedule's host passes need only the
     // permuted CSR structure and the levels, so they run on a thread while
-    // steps 4-8 run; the upload follows step 8
+    // steps 4-8 run; the upload follows step 8.  It is made for rows of few
+    // entries, most of them in the wave's previous step; for longer rows the
+    // level schedule is built first, and alone where it is clearly faster.
+    const bool level_first = p->want_schedule == RB_SCHED_AUTO && nnz > 4L * m;
     FusedJob *fjob = nullptr;
     struct JobGuard {  // an early return abandons the job (joins the thread)
         FusedJob *&j;
@@ -582,10 +586,17 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
             if (j) (void)build_fused_finish(j, false);
         }
     } jguard{fjob};
-    auto t_fs0 = std::chrono::steady_clock::now();
-    if (p->want_schedule != RB_SCHED_BLOCKED && m > 0)
-        RB_TRY(build_fused_start(p, prptr, ccol, cval, p->fused_waves, s, &fjob));
-    auto t_fs1 = std::chrono::steady_clock::now();
+    double fused_ms = 0.0;
+    auto start_fused = [&]() -> rb_status {
+        auto t = std::chrono::steady_clock::now();
+        if (p->want_schedule != RB_SCHED_BLOCKED && m > 0)
+            RB_TRY(build_fused_start(p, prptr, ccol, cval, p->fused_waves, s, &fjob));
+        fused_ms = std::chrono::duration<double, std::milli>(
+                       std::chrono::steady_clock::now() - t)
+                       .count();
+        return RB_OK;
+    };
+    if (!level_first) RB_TRY(start_fused());
     mark("csr");
     // ---- 4. partition and slot space
     p->ntri = 1 << p->lv;
@@ -633,6 +644,10 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
                                            p->d_rowptr, p->d_col, p->d_val);
     RB_HIP(hipGetLastError());
 
+    if (level_first) {
+        RB_TRY(build_level(p, prptr, ccol, cval, s));
+        if (!level_beats_chain(p)) RB_TRY(start_fused());
+    }
     mark("slots");
     // ---- 5. block statistics (blk_nnz, cal_longrow)
     int *d_stats;
@@ -831,6 +846,12 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     auto t_f1 = std::chrono::steady_clock::now();
 
     mark("fused");
+    if (p->want_schedule == RB_SCHED_AUTO && !level_first && m > 0) {
+        bool narrow = !p->fused;
+        if (!narrow) RB_TRY(level_narrow(p, s, &narrow));
+        if (narrow) RB_TRY(build_level(p, prptr, ccol, cval, s));
+    }
+    mark("level");
     // ---- 10. FP32 + FP64-refinement storage: FP32 copies of the slot
     // values, and the original matrix as CSR for the FP64 residuals (rows,
     // b, r and the x gathers all in the caller's order: the level-ordered
@@ -877,7 +898,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     p->phase_ms[0] = ms(t0, t_lv);
     // the fused build's own share: structure copies, then the wait for its
     // host passes and the upload (the passes overlap steps 4-8)
-    p->phase_ms[2] = ms(t_fs0, t_fs1) + ms(t_f0, t_f1);
+    p->phase_ms[2] = fused_ms + ms(t_f0, t_f1);
     p->phase_ms[1] = p->preprocess_ms - p->phase_ms[0] - p->phase_ms[2];
     mark("scratch");
     if (trace) {

@@ -929,7 +929,7 @@ void rowcap_for_call(rb_plan *p, hipStream_t s) {
 
 // Right-hand sides one walk takes: up to 32, within 4 GiB of permuted b
 // and x (32 columns up to 8M rows).
-static int walk_cols(const rb_plan *p) {
+int walk_cols(const rb_plan *p) {
     const long per = 16L * std::max(1, p->m);
     return (int)std::max(1L, std::min(32L, (4L << 30) / per));
 }
@@ -981,6 +981,10 @@ static rb_status ensure_cols(rb_plan *p, int ncol, hipStream_t s) {
     }
     cap = ncol;
     return RB_OK;
+}
+
+rb_status scratch_cols(rb_plan *p, int ncol, hipStream_t s) {
+    return ensure_cols<double>(p, walk_width(p, ncol), s);
 }
 
 template <class T>
@@ -1299,7 +1303,10 @@ rb_status solve_f32ir(rb_plan *p, const double *d_b, int ldb, double *d_x,
             // once every column has converged the solve is skipped (the
             // walk's prologue sets the width its kernels read to zero; the
             // fused kernels return at once)
-            if (p->schedule == RB_SCHED_FUSED && p->fused) {
+            if (p->use_level) {
+                RB_TRY(solve_level32(p, p->d_r, m, x, ldx, nc, s, p->d_irleft,
+                                     p->d_irdone));
+            } else if (p->schedule == RB_SCHED_FUSED && p->fused) {
                 // rounding of r, the solve and x += d in the fused passes
                 RB_TRY(solve_fused32(p, p->d_r, m, x, ldx, nc, s, p->d_irleft,
                                      p->d_irdone));
