@@ -140,14 +140,14 @@ rb_status canonicalize_csc(const int *d_colptr, const int *d_rowidx,
     RB_HIP(hipGetLastError());
     const int bits = bits_for(n);
     // stable by row, then stable by column: (column, row, input position)
-    RB_TRY(sort_pairs_i32(d_rowidx, row1, iota, idx1, nnz, bits, s));
+    RB_TRY(sort_pairs_i32(d_rowidx, row1, iota, idx1, nnz, bits, s, tmp));
     k_canon_gather<<<nblk(nnz), kT, 0, s>>>(ecol, idx1, nnz, key2);
     RB_HIP(hipGetLastError());
-    RB_TRY(sort_pairs_i32(key2, col2, idx1, idx2, nnz, bits, s));
+    RB_TRY(sort_pairs_i32(key2, col2, idx1, idx2, nnz, bits, s, tmp));
     k_canon_gather<<<nblk(nnz), kT, 0, s>>>(d_rowidx, idx2, nnz, row2);
     k_canon_heads<<<nblk(nnz), kT, 0, s>>>(col2, row2, nnz, head);
     RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(head, pos, nnz, s));
+    RB_TRY(exclusive_scan_i32(head, pos, nnz, s, tmp));
     int last[2];
     RB_HIP(hipMemcpyAsync(&last[0], pos + nnz - 1, sizeof(int), hipMemcpyDeviceToHost, s));
     RB_HIP(hipMemcpyAsync(&last[1], head + nnz - 1, sizeof(int), hipMemcpyDeviceToHost, s));
@@ -158,7 +158,7 @@ rb_status canonicalize_csc(const int *d_colptr, const int *d_rowidx,
     k_canon_merge<<<nblk(nnz), kT, 0, s>>>(col2, row2, idx2, d_val, head, pos, nnz,
                                            *c_rowidx, *c_val, colcnt);
     RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(colcnt, *c_colptr, n + 1, s));
+    RB_TRY(exclusive_scan_i32(colcnt, *c_colptr, n + 1, s, tmp));
     *c_nnz = nu;
     return RB_OK;
 }

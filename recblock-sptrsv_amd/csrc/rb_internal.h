@@ -84,12 +84,12 @@ struct Arena {
 
 // Device-wide primitives (rb_prim.hip, hipCUB).
 rb_status exclusive_scan_i32(const int *d_in, int *d_out, int n,
-                             hipStream_t s);
+                             hipStream_t s, Arena &tmp);
 rb_status inclusive_max_i32(const int *d_in, int *d_out, int n,
-                            hipStream_t s);
+                            hipStream_t s, Arena &tmp);
 rb_status sort_pairs_i32(const int *keys_in, int *keys_out,
                          const int *vals_in, int *vals_out, int n, int bits,
-                         hipStream_t s);
+                         hipStream_t s, Arena &tmp);
 
 // Level analysis: Kahn BFS in the reference's discovery order
 // (rb_levels.hip).  colptr/rowidx: square CSC whose columns hold the
@@ -313,8 +313,31 @@ rb_status solve_level_batch(rb_plan *p, const double *const *d_b, double *const 
 // right-hand sides one pass over the columns takes; permuted b / x scratch
 // for ncol of them
 int walk_cols(const rb_plan *p);
+int walk_launches(const rb_plan *p);  // kernels of the blocked walk
 rb_status scratch_cols(rb_plan *p, int ncol, hipStream_t s);
 void level_destroy(rb_plan *p);
+// do n columns at b overlap n columns at x other than being the same?
+inline bool part_overlap(const double *b, long ldb, const double *x, long ldx, int m, int n) {
+    if (b == x && (ldb == ldx || n == 1)) return false;
+    return b < x + (n - 1) * ldx + m && x < b + (n - 1) * ldb + m;
+}
+// Every entry [a, b) of every lane's row, f(k, v...) with v the row's values;
+// called by whole waves.  A row of more than 32 entries is taken by its wave:
+// one thread alone goes through it entry by entry (21,527 power-law rows, the
+// longest of 508: 347 us for a pass over all entries, 101 like this).
+template <class F, class... V>
+__device__ inline void each_entry(int a, int b, F f, V... v) {
+    const bool wide = b - a > 32;
+    if (!wide)
+        for (int k = a; k < b; k++) f(k, v...);
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int l = __ffsll(todo) - 1;
+        const int la = __shfl(a, l, 64), lb = __shfl(b, l, 64);
+        [&](V... w) {
+            for (int k = la + (int)(threadIdx.x & 63); k < lb; k += 64) f(k, w...);
+        }(__shfl(v, l, 64)...);
+    }
+}
 size_t level_bytes(const rb_plan *p);
 // the same solves on caller-provided per-solve buffers (ws, ws_bytes)
 // instead of the plan's: the blocked walk needs blocked_ws_bytes(p) (one

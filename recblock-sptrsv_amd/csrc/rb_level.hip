@@ -430,15 +430,18 @@ __global__ void k_lv_own(RowGeom g, const int *__restrict__ rp, const int *__res
     if ((threadIdx.x & 63) == 0 && len > 0) atomicMax(longest, len);
 }
 
+// the first level that needs a row's x
 __global__ void k_lv_need(int m, const int *__restrict__ rp, const int *__restrict__ cc,
                           const int *__restrict__ level, int *need) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= m) return;
-    const int l = level[r];
-    for (int k = rp[r]; k < rp[r + 1]; k++) {
-        int *at = need + cc[k];
-        if (cc[k] != r && *(volatile int *)at > l) atomicMin(at, l);
-    }
+    const bool live = r < m;
+    each_entry(
+        live ? rp[r] : 0, live ? rp[r + 1] : 0,
+        [&](int k, int row, int l) {
+            int *at = need + cc[k];
+            if (cc[k] != row && *(volatile int *)at > l) atomicMin(at, l);
+        },
+        r, live ? level[r] : 0);
 }
 
 __global__ void k_lv_block_start(int m, const int *__restrict__ level,
@@ -501,25 +504,29 @@ __global__ void k_lv_blocks(const int *__restrict__ key, const int *__restrict__
                             const int *__restrict__ off, const int *__restrict__ blk0,
                             int *first_c, int *last_c, int *first_p, int *last_p) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g.m) return;
-    const int r = g.fwd ? order[i] : g.m - 1 - order[i];
-    const int p = (key[i] >> 3) / g.nlev, l = (key[i] >> 3) - p * g.nlev;
-    const int o = off ? off[p] : 0, b0 = blk0[p];
+    const bool live = i < g.m;
+    const int r = !live ? 0 : g.fwd ? order[i] : g.m - 1 - order[i];
+    const int pl = live ? key[i] >> 3 : 0, p = pl / g.nlev;
     // (the plain read first: most atomics would change nothing)
-    auto low = [&](int *a, int u) {
-        int *at = a + b0 + (u - o) / kBlock;
+    if (live) {
+        const int l = pl - p * g.nlev, o = off ? off[p] : 0;
+        int *at = first_c + blk0[p] + (lf[r] - o) / kBlock;
         if (*(volatile int *)at > l) atomicMin(at, l);
-    };
-    auto high = [&](int *a, int u) {
-        int *at = a + b0 + (u - o) / kBlock;
-        if (*(volatile int *)at < l) atomicMax(at, l);
-    };
-    low(first_c, lf[r]);
-    low(first_p, i);
-    for (int k = rp[r]; k < rp[r + 1]; k++) {  // (the diagonal: the row itself)
-        high(last_c, lf[cc[k]]);
-        high(last_p, newpos[cc[k]]);
+        // (levels rise with the position)
+        if ((i - o) % kBlock == 0) first_p[blk0[p] + (i - o) / kBlock] = l;
     }
+    // (the diagonal: the row itself)
+    each_entry(
+        live ? rp[r] : 0, live ? rp[r + 1] : 0,
+        [&](int k, int q, int l) {
+            const int o = off ? off[q] : 0, b0 = blk0[q];
+            auto high = [&](int *at) {
+                if (*(volatile int *)at < l) atomicMax(at, l);
+            };
+            high(last_c + b0 + (lf[cc[k]] - o) / kBlock);
+            high(last_p + b0 + (newpos[cc[k]] - o) / kBlock);
+        },
+        p, pl - p * g.nlev);
 }
 
 // empty lanes: no row, coefficients 0 on the ring's zero
@@ -713,7 +720,7 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
         return np == 1 && level_us(p, nsteps) > 8.0 * chain_us(p);
     };
     if (too_wide(m / 64)) return RB_OK;
-    Arena tmp(56 * (size_t)m + (1 << 20));
+    Arena tmp(76 * (size_t)m + (1 << 20));
     struct Guard {
         Arena &a;
         ~Guard() { a.release(); }
@@ -735,14 +742,14 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
     k_lv_key<<<nblk(m), kT, 0, s>>>(g, d_rp, lev, newpos, rend, p->d_levelItem, p->d_part, k0,
                                     v0);
     RB_HIP(hipGetLastError());
-    RB_TRY(sort_pairs_i32(k0, key, v0, order, m, bits_for((long)np * p->nlevel * 8), s));
+    RB_TRY(sort_pairs_i32(k0, key, v0, order, m, bits_for((long)np * p->nlevel * 8), s, tmp));
     k_lv_heads<<<nblk(m), kT, 0, s>>>(key, m, k0, v0);
     RB_HIP(hipGetLastError());
-    RB_TRY(inclusive_max_i32(k0, run, m, s));
-    RB_TRY(inclusive_max_i32(v0, lev, m, s));
+    RB_TRY(inclusive_max_i32(k0, run, m, s, tmp));
+    RB_TRY(inclusive_max_i32(v0, lev, m, s, tmp));
     k_lv_steps<<<nblk(m), kT, 0, s>>>(key, run, lev, order, g, head, rend, newpos);
     RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(head, sidx, m + 1, s));
+    RB_TRY(exclusive_scan_i32(head, sidx, m + 1, s, tmp));
     // the parts' rows and blocks
     std::vector<Part> parts(np);
     std::vector<int> blk0(np + 1, 0);
@@ -855,12 +862,6 @@ static rb_status launch_level(rb_plan *p, const LevelArgs<T> &a, int grid, hipSt
     RB_HIP(hipGetLastError());
     mark_end(p, s);
     return RB_OK;
-}
-
-// Does [b] overlap [x] other than being it?
-static bool part_overlap(const double *b, long ldb, const double *x, long ldx, int m, int n) {
-    if (b == x && (ldb == ldx || n == 1)) return false;
-    return b < x + (n - 1) * ldx + m && x < b + (n - 1) * ldb + m;
 }
 
 // nc columns; sb: scratch in storage order (m per column), unless the storage

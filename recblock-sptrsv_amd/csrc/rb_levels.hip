@@ -25,7 +25,10 @@ namespace rb {
 
 namespace {
 
-constexpr int kBfsThreads = 256;
+// (256 and 1024 threads: 300,001 power-law rows backward 11.1 and 6.6 ms,
+// 21,527 forward 1.8 and 1.2, 250,000 rows of a grid 5.6 and 5.5)
+constexpr int kBfsThreads = 1024, kBfsWaves = kBfsThreads / 64;
+constexpr int kScan = kBfsWaves + 2;  // ints of LDS for a scan
 
 struct BfsCtl {
     int s, e;     // current frontier [s, e) of levelItem
@@ -33,9 +36,10 @@ struct BfsCtl {
     int stalled;  // 1 when a round adds nothing while rows remain
 };
 
-// Exclusive scan of one value per thread across a 256-thread block.
-// Returns the exclusive prefix; *total receives the block sum.
-__device__ inline int block_excl_scan(int v, int *lds, int *total) {
+// Exclusive scan of one value per thread across the block.  Returns the
+// exclusive prefix; *total receives the block sum.  lds may be written again
+// after the next barrier.
+__device__ inline int block_excl_scan_open(int v, int *lds, int *total) {
     const int lane = threadIdx.x & 63;
     const int wid = threadIdx.x >> 6;
     int x = v;
@@ -46,20 +50,20 @@ __device__ inline int block_excl_scan(int v, int *lds, int *total) {
     }
     if (lane == 63) lds[wid] = x;
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int w = 0; w < kBfsThreads / 64; w++) {
-            int t = lds[w];
-            lds[w] = run;
-            run += t;
-        }
-        lds[kBfsThreads / 64] = run;
+    // every wave scans the waves' sums for itself
+    int w = lane < kBfsWaves ? lds[lane] : 0;
+#pragma unroll
+    for (int o = 1; o < kBfsWaves; o <<= 1) {
+        int y = __shfl_up(w, o, 64);
+        if (lane >= o) w += y;
     }
+    *total = __shfl(w, kBfsWaves - 1, 64);
+    return x - v + (wid > 0 ? __shfl(w, wid - 1, 64) : 0);
+}
+__device__ inline int block_excl_scan(int v, int *lds, int *total) {
+    const int r = block_excl_scan_open(v, lds, total);
     __syncthreads();
-    int res = x - v + lds[wid];
-    *total = lds[kBfsThreads / 64];
-    __syncthreads();
-    return res;
+    return r;
 }
 
 __device__ inline int ld_relaxed(const int *p) {
@@ -96,11 +100,11 @@ __device__ int grid_excl_scan(cg::grid_group &g, int *cnt, int len,
             int v = i < G ? ld_relaxed(&blocksum[i]) : 0;
             int t;
             int ex = block_excl_scan(v, lds, &t);
-            if (i == blockIdx.x) lds[8] = run + ex;
+            if (i == blockIdx.x) lds[kBfsWaves] = run + ex;
             run += t;
             __syncthreads();
         }
-        before = lds[8];
+        before = lds[kBfsWaves];
         grand = run;
         __syncthreads();
     }
@@ -118,99 +122,195 @@ __device__ int grid_excl_scan(cg::grid_group &g, int *cnt, int len,
 }
 
 constexpr int kNarrow = 4096;  // frontier size handled by one workgroup
-constexpr int kIlp = 6;        // frontier nodes per thread, cached levels
+constexpr int kIlp = 2;        // frontier nodes per thread, cached levels
 constexpr int kE = 4;          // column entries per node kept in registers
 
-// Exclusive scan of cl[0..len) in place (one workgroup); returns the sum.
-__device__ int narrow_scan(int *cl, int len, int *lds) {
-    const int tid = threadIdx.x;
-    const int per = (len + blockDim.x - 1) / blockDim.x;
-    const int lo = min(len, tid * per), hi = min(len, lo + per);
-    int local = 0;
-    for (int i = lo; i < hi; i++) local += cl[i];
-    int total;
-    int run = block_excl_scan(local, lds, &total);
-    for (int i = lo; i < hi; i++) {
-        const int t = cl[i];
-        cl[i] = run;
-        run += t;
-    }
-    __syncthreads();
-    return total;
+// The phases over the entries [a, b) of a node's column (node u at position
+// p).  Thread by thread, four entries in flight, or by a whole wave (with
+// uniform arguments), 64 entries at a time, for a column of more than
+// kLongCol entries: one thread alone needs two trips to memory for every four
+// of them, and power-law factors have columns of thousands (300,001 rows
+// backward: 47 ms with one thread and one entry at a time, 6.6 like this).
+constexpr int kLongCol = 16;
+constexpr int kWg = __HIP_MEMORY_SCOPE_WORKGROUP, kDev = __HIP_MEMORY_SCOPE_AGENT;
+constexpr auto kCount = [](int, int) {};
+
+template <int SC>
+__device__ inline int ld_sc(const int *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, SC);
 }
 
-// The frontier of the next level, kept in LDS by a cached level when that
-// level is cached too: its nodes and their column ranges [a, b).
+// A: decrement dependants, raise their parent position
+template <int SC>
+__device__ inline void release(int v, int *rem, int *par, int u, int p) {
+    if (v == u) return;
+    __hip_atomic_fetch_add(&rem[v], -1, __ATOMIC_RELAXED, SC);
+    __hip_atomic_fetch_max(&par[v], p, __ATOMIC_RELAXED, SC);
+}
+
+// The children (rem 0, parent p), in column order: B counts them (put does
+// nothing), C puts child v at o, o + 1, ...  Returns their number.
+template <int SC, class Put>
+__device__ inline int children(const int *__restrict__ rowidx, const int *rem, const int *par,
+                               int a, int b, int u, int p, int o, Put put) {
+    int c = 0;
+    for (int q = a; q < b; q += 4) {
+        int v[4], r[4], t[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = q + j < b ? rowidx[q + j] : u;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            r[j] = ld_sc<SC>(&rem[v[j]]);
+            t[j] = ld_sc<SC>(&par[v[j]]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (v[j] != u && r[j] == 0 && t[j] == p) put(o + c++, v[j]);
+    }
+    return c;
+}
+template <int SC, class Put>
+__device__ inline int wave_children(const int *__restrict__ rowidx, const int *rem,
+                                    const int *par, int a, int b, int u, int p, int o, Put put) {
+    const int lane = threadIdx.x & 63;
+    int n = 0;
+    for (int q = a; q < b; q += 64) {
+        const int v = q + lane < b ? rowidx[q + lane] : u;
+        const int r = ld_sc<SC>(&rem[v]), t = ld_sc<SC>(&par[v]);
+        const bool kid = v != u && r == 0 && t == p;
+        const unsigned long long kids = __ballot(kid);
+        if (kid) put(o + n + __popcll(kids & ((1ull << lane) - 1)), v);
+        n += __popcll(kids);
+    }
+    return n;
+}
+
+// The same for every lane's node at once (a == b: none), called by whole
+// waves: short columns thread by thread, then the long ones one by one.
+template <int SC>
+__device__ inline void each_release(const int *__restrict__ rowidx, int *rem, int *par, int a,
+                                    int b, int u, int p) {
+    const bool wide = b - a > kLongCol;
+    if (!wide)
+        for (int q = a; q < b; q++) release<SC>(rowidx[q], rem, par, u, p);
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int l = __ffsll(todo) - 1;
+        const int la = __shfl(a, l, 64), lb = __shfl(b, l, 64);
+        const int lu = __shfl(u, l, 64), lp = __shfl(p, l, 64);
+        for (int q = la + (threadIdx.x & 63); q < lb; q += 64)
+            release<SC>(rowidx[q], rem, par, lu, lp);
+    }
+}
+template <int SC, class Put>
+__device__ inline int each_children(const int *__restrict__ rowidx, const int *rem,
+                                    const int *par, int a, int b, int u, int p, int o, Put put) {
+    const bool wide = b - a > kLongCol;
+    int c = 0;
+    if (!wide) c = children<SC>(rowidx, rem, par, a, b, u, p, o, put);
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int l = __ffsll(todo) - 1;
+        const int n = wave_children<SC>(rowidx, rem, par, __shfl(a, l, 64), __shfl(b, l, 64),
+                                        __shfl(u, l, 64), __shfl(p, l, 64), __shfl(o, l, 64),
+                                        put);
+        if ((int)(threadIdx.x & 63) == l) c = n;
+    }
+    return c;
+}
+
+// A level's frontier in LDS, left there by a cached level for the next when
+// that is cached too: its nodes and their column ranges [a, b).
 struct Front {
     int u[kIlp * kBfsThreads];
     int a[kIlp * kBfsThreads];
     int b[kIlp * kBfsThreads];
 };
+struct Walk {
+    Front fr[2];
+    int nlong;                        // nodes with long columns ...
+    int node[kIlp * kBfsThreads];     // ... which they are
+    int kids[kIlp * kBfsThreads];     // ... and their children: how many, then where
+    int lds[kScan];
+};
 
-// One narrow level [s, e) of at most kIlp * kBfsThreads nodes.  Each thread
-// keeps its nodes, their entry ranges and the first kE entries of their
-// columns in registers from phase A to C, and phase B remembers which of
-// those entries are children, so B reads only rem / par and C only writes:
-// a level costs about four dependent memory round trips instead of a dozen.
-// Entries past the first kE of a column are re-read (the generic rule).
-__device__ int level_cached(const int *__restrict__ colptr,
-                            const int *__restrict__ rowidx, int *rem, int *par,
-                            int *levelItem, int s, int e, int *cl, int *lds,
-                            Front &fr, bool &held) {
-    const int tid = threadIdx.x, len = e - s;
-    const bool in = held;  // this level's nodes and column ranges are in fr
-    int u[kIlp], q0[kIlp], q1[kIlp], vc[kIlp][kE];
-    unsigned kid[kIlp];
-    if (in) {
+// One narrow level [s, e) of at most N * kBfsThreads nodes, N to a thread.
+// Each thread keeps its nodes, their entry ranges and the first kE entries of
+// their columns in registers from phase A to C, and phase B remembers which
+// of those entries are children, so B reads only rem / par and C only writes.
+// Entries past the first kE are re-read in each phase, by the thread or, in a
+// long column, by the next wave that is free: the nodes with long columns are
+// listed in LDS (the first levels of a power-law factor hold most of them).
+// N is 1 where the level fits: places without a node still cost the loads of
+// phase B (250 nodes a level, 256 threads: 7.3 us with six places, 5.6 with
+// one).
+template <int N>
+__device__ int level_cached_n(const int *__restrict__ colptr, const int *__restrict__ rowidx,
+                              int *rem, int *par, int *levelItem, int s, int e, Walk &w,
+                              int &held) {
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, len = e - s;
+    const bool in = held >= 0;  // this level's nodes and column ranges are in cur
+    const int c0 = in ? held : 0;
+    Front &cur = w.fr[c0], &fr = w.fr[c0 ^ 1];
+    int u[N], q0[N], q1[N], vc[N][kE], at[N];
+    unsigned kid[N];
 #pragma unroll
-        for (int k = 0; k < kIlp; k++) {
-            const int i = tid + k * kBfsThreads;
-            u[k] = i < len ? fr.u[i] : -1;
-            q0[k] = i < len ? fr.a[i] : 0;
-            q1[k] = i < len ? fr.b[i] : 0;
-        }
-    } else {
+    for (int k = 0; k < N; k++) {
+        const int i = tid * N + k;
+        u[k] = i >= len ? -1 : in ? cur.u[i] : ld_wg(&levelItem[s + i]);
+    }
 #pragma unroll
-        for (int k = 0; k < kIlp; k++) {
-            const int i = tid + k * kBfsThreads;
-            u[k] = i < len ? ld_wg(&levelItem[s + i]) : -1;
-        }
-#pragma unroll
-        for (int k = 0; k < kIlp; k++) {
-            q0[k] = u[k] >= 0 ? colptr[u[k]] : 0;
-            q1[k] = u[k] >= 0 ? colptr[u[k] + 1] : 0;
+    for (int k = 0; k < N; k++) {
+        const int i = tid * N + k;
+        q0[k] = u[k] < 0 ? 0 : in ? cur.a[i] : colptr[u[k]];
+        q1[k] = u[k] < 0 ? 0 : in ? cur.b[i] : colptr[u[k] + 1];
+        if (!in && i < len) {
+            cur.u[i] = u[k];
+            cur.a[i] = q0[k];
+            cur.b[i] = q1[k];
         }
     }
 #pragma unroll
-    for (int k = 0; k < kIlp; k++)
+    for (int k = 0; k < N; k++)
 #pragma unroll
         for (int j = 0; j < kE; j++)
             vc[k][j] = q0[k] + j < q1[k] ? rowidx[q0[k] + j] : -1;
+    auto is_long = [&](int k) { return q1[k] - q0[k] > kLongCol; };
     // A: decrement dependants, raise their parent position
 #pragma unroll
-    for (int k = 0; k < kIlp; k++) {
-        const int p = s + tid + k * kBfsThreads;
+    for (int k = 0; k < N; k++) {
+        const int p = s + tid * N + k;
 #pragma unroll
-        for (int j = 0; j < kE; j++) {
-            const int v = vc[k][j];
-            if (v < 0 || v == u[k]) continue;
-            __hip_atomic_fetch_add(&rem[v], -1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_max(&par[v], p, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-        for (int q = q0[k] + kE; q < q1[k]; q++) {
-            const int v = rowidx[q];
-            if (v == u[k]) continue;
-            __hip_atomic_fetch_add(&rem[v], -1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_max(&par[v], p, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+        for (int j = 0; j < kE; j++)
+            if (vc[k][j] >= 0) release<kWg>(vc[k][j], rem, par, u[k], p);
+        if (is_long(k)) {
+            at[k] = __hip_atomic_fetch_add(&w.nlong, 1, __ATOMIC_RELAXED, kWg);
+            w.node[at[k]] = tid * N + k;
+        } else {
+            for (int q = q0[k] + kE; q < q1[k]; q++) release<kWg>(rowidx[q], rem, par, u[k], p);
         }
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    auto fence = [] {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    };
+    fence();
+    const int nlong = w.nlong;
+    if (nlong > 0) {
+        for (int g = wave; g < nlong; g += kBfsWaves) {
+            const int i = w.node[g], b = cur.b[i], uu = cur.u[i];
+            for (int q = cur.a[i] + kE + lane; q < b; q += 64)
+                release<kWg>(rowidx[q], rem, par, uu, s + i);
+        }
+        fence();
+        if (tid == 0) w.nlong = 0;
+        for (int g = wave; g < nlong; g += kBfsWaves) {
+            const int i = w.node[g];
+            const int n = wave_children<kWg>(rowidx, rem, par, cur.a[i] + kE, cur.b[i], cur.u[i],
+                                             s + i, 0, kCount);
+            if (lane == 0) w.kids[g] = n;
+        }
+        __syncthreads();
+    }
     // B: children (rem 0, parent p) per node.  The cached entries' rem and
     // par are read together (a non-candidate reads row 0, in range, and is
     // ignored), and with them the entries' column ranges, which a child
@@ -219,9 +319,9 @@ __device__ int level_cached(const int *__restrict__ colptr,
     // entries, atomics, rem / par) at ~2 us each on the 1500^2 Laplacian;
     // with the frontier in LDS three are left.  Reading rem / par entry by
     // entry behind branches cost another ~0.5 us.
-    int rv[kIlp][kE], pv[kIlp][kE], ca[kIlp][kE], cb[kIlp][kE];
+    int rv[N][kE], pv[N][kE], ca[N][kE], cb[N][kE];
 #pragma unroll
-    for (int k = 0; k < kIlp; k++)
+    for (int k = 0; k < N; k++)
 #pragma unroll
         for (int j = 0; j < kE; j++) {
             const int v = vc[k][j];
@@ -231,10 +331,10 @@ __device__ int level_cached(const int *__restrict__ colptr,
             ca[k][j] = colptr[va];
             cb[k][j] = colptr[va + 1];
         }
+    int cnt[N], own = 0;
 #pragma unroll
-    for (int k = 0; k < kIlp; k++) {
-        const int i = tid + k * kBfsThreads;
-        const int p = s + i;
+    for (int k = 0; k < N; k++) {
+        const int p = s + tid * N + k;
         int c = 0;
         unsigned bits = 0;
 #pragma unroll
@@ -246,122 +346,125 @@ __device__ int level_cached(const int *__restrict__ colptr,
                 bits |= 1u << j;
             }
         }
-        for (int q = q0[k] + kE; q < q1[k]; q++) {
-            const int v = rowidx[q];
-            if (v != u[k] && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p) c++;
-        }
+        if (is_long(k)) c += w.kids[at[k]];
+        else c += children<kWg>(rowidx, rem, par, q0[k] + kE, q1[k], u[k], p, 0, kCount);
         kid[k] = bits;
-        if (i < len) cl[i] = c;
+        cnt[k] = c;
+        own += c;
     }
-    __syncthreads();
-    const int total = narrow_scan(cl, len, lds);
+    int total;
+    int o = e + block_excl_scan_open(own, w.lds, &total);
     // C: children in column order at the node's offset; when the next
-    // level is cached too, its frontier also goes to fr (every read of fr
-    // was in A, before this level's barriers)
+    // level is cached too, its frontier also goes to the other fr
     const bool out = total <= kIlp * kBfsThreads;
+    auto put = [&](int to, int v) {
+        if (out) {
+            fr.u[to - e] = v;
+            fr.a[to - e] = colptr[v];
+            fr.b[to - e] = colptr[v + 1];
+        }
+        __hip_atomic_store(&levelItem[to], v, __ATOMIC_RELAXED, kWg);
+    };
 #pragma unroll
-    for (int k = 0; k < kIlp; k++) {
-        const int i = tid + k * kBfsThreads;
-        if (i >= len) continue;
-        const int p = s + i;
-        int o = e + cl[i];
+    for (int k = 0; k < N; k++) {
+        const int p = s + tid * N + k;
+        int to = o;
 #pragma unroll
         for (int j = 0; j < kE; j++)
             if ((kid[k] >> j) & 1u) {
                 if (out) {
-                    fr.u[o - e] = vc[k][j];
-                    fr.a[o - e] = ca[k][j];
-                    fr.b[o - e] = cb[k][j];
+                    fr.u[to - e] = vc[k][j];
+                    fr.a[to - e] = ca[k][j];
+                    fr.b[to - e] = cb[k][j];
                 }
-                __hip_atomic_store(&levelItem[o++], vc[k][j], __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
+                __hip_atomic_store(&levelItem[to++], vc[k][j], __ATOMIC_RELAXED, kWg);
             }
-        for (int q = q0[k] + kE; q < q1[k]; q++) {
-            const int v = rowidx[q];
-            if (v != u[k] && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p) {
-                if (out) {
-                    fr.u[o - e] = v;
-                    fr.a[o - e] = colptr[v];
-                    fr.b[o - e] = colptr[v + 1];
-                }
-                __hip_atomic_store(&levelItem[o++], v, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
+        if (is_long(k)) w.kids[at[k]] = to;
+        else children<kWg>(rowidx, rem, par, q0[k] + kE, q1[k], u[k], p, to, put);
+        o += cnt[k];
+    }
+    if (nlong > 0) {
+        __syncthreads();
+        for (int g = wave; g < nlong; g += kBfsWaves) {
+            const int i = w.node[g];
+            wave_children<kWg>(rowidx, rem, par, cur.a[i] + kE, cur.b[i], cur.u[i], s + i,
+                               w.kids[g], put);
         }
     }
-    held = out;
+    held = out ? c0 ^ 1 : -1;
     return total;
 }
+__device__ int level_cached(const int *__restrict__ colptr, const int *__restrict__ rowidx,
+                            int *rem, int *par, int *levelItem, int s, int e, Walk &w,
+                            int &held) {
+    static_assert(kIlp == 2);
+    if (e - s <= kBfsThreads)
+        return level_cached_n<1>(colptr, rowidx, rem, par, levelItem, s, e, w, held);
+    return level_cached_n<2>(colptr, rowidx, rem, par, levelItem, s, e, w, held);
+}
 
-// One narrow level of any width up to kNarrow: the same phases, each
-// re-reading the frontier's columns.
-__device__ int level_generic(const int *__restrict__ colptr,
-                             const int *__restrict__ rowidx, int *rem, int *par,
-                             int *levelItem, int s, int e, int *cl, int *lds) {
-    const int tid = threadIdx.x, len = e - s;
-    for (int p = s + tid; p < e; p += blockDim.x) {
-        const int u = ld_wg(&levelItem[p]);
-        for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-            const int v = rowidx[q];
-            if (v == u) continue;
-            __hip_atomic_fetch_add(&rem[v], -1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_max(&par[v], p, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
+// One level [s, e) of any width inside one workgroup: the A / B / scan /
+// C phases of the narrow levels, with the counts in device memory (cnt,
+// indexed by frontier position) and a scan in chunks of the workgroup's
+// width.  A thread handles the same positions in B and C, so it reads back
+// only its own counts.
+__device__ int level_wide(const int *__restrict__ colptr,
+                          const int *__restrict__ rowidx, int *rem, int *par,
+                          int *levelItem, int s, int e, int *cnt, int *lds) {
+    const int tid = threadIdx.x;
+    for (int base = s; base < e; base += blockDim.x) {  // uniform trip counts
+        const int p = base + tid;
+        const int u = p < e ? ld_wg(&levelItem[p]) : -1;
+        each_release<kWg>(rowidx, rem, par, u >= 0 ? colptr[u] : 0, u >= 0 ? colptr[u + 1] : 0,
+                         u, p);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
     __syncthreads();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    for (int i = tid; i < len; i += blockDim.x) {
-        const int p = s + i;
-        const int u = ld_wg(&levelItem[p]);
-        int c = 0;
-        for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-            const int v = rowidx[q];
-            if (v != u && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p) c++;
-        }
-        cl[i] = c;
+    int carry = 0;
+    for (int base = s; base < e; base += blockDim.x) {
+        const int p = base + tid;
+        const int u = p < e ? ld_wg(&levelItem[p]) : -1;
+        const int c = each_children<kWg>(rowidx, rem, par, u >= 0 ? colptr[u] : 0,
+                                    u >= 0 ? colptr[u + 1] : 0, u, p, 0, kCount);
+        int tot = 0;
+        const int off = block_excl_scan(c, lds, &tot);
+        if (p < e) cnt[p] = carry + off;
+        carry += tot;
     }
-    __syncthreads();
-    const int total = narrow_scan(cl, len, lds);
-    for (int i = tid; i < len; i += blockDim.x) {
-        const int p = s + i;
-        const int u = ld_wg(&levelItem[p]);
-        int o = e + cl[i];
-        for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-            const int v = rowidx[q];
-            if (v != u && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p)
-                __hip_atomic_store(&levelItem[o++], v, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
+    for (int base = s; base < e; base += blockDim.x) {
+        const int p = base + tid;
+        const int u = p < e ? ld_wg(&levelItem[p]) : -1;
+        each_children<kWg>(rowidx, rem, par, u >= 0 ? colptr[u] : 0, u >= 0 ? colptr[u + 1] : 0, u,
+                      p, p < e ? e + cnt[p] : e, [&](int at, int v) {
+                          __hip_atomic_store(&levelItem[at], v, __ATOMIC_RELAXED, kWg);
+                      });
     }
-    return total;
+    return carry;
 }
 
 // Consecutive narrow levels inside workgroup 0: the same A / B / scan / C
-// phases, separated by workgroup barriers.  Frontier counts live in LDS.
-// rem / par / levelItem are read, updated and written at workgroup scope
-// (see ld_wg).
+// phases, separated by workgroup barriers.  rem / par / levelItem are read,
+// updated and written at workgroup scope (see ld_wg).
 __device__ void bfs_narrow(const int *__restrict__ colptr,
                            const int *__restrict__ rowidx, int m, int *rem,
-                           int *par, int *levelItem, int *levelPtr,
-                           BfsCtl *ctl, int *lds) {
-    __shared__ int cl[kNarrow];
-    __shared__ Front fr;
+                           int *par, int *cnt, int *levelItem, int *levelPtr,
+                           BfsCtl *ctl) {
+    __shared__ Walk w;
     const int tid = threadIdx.x;
+    if (tid == 0) w.nlong = 0;
+    __syncthreads();
     int s = ld_relaxed(&ctl->s), e = ld_relaxed(&ctl->e);
     int nl = ld_relaxed(&ctl->nlevel);
     int stalled = 0;
-    bool held = false;  // the level's frontier is in fr
+    int held = -1;  // which of w.fr holds the level's frontier, -1: neither
     while (e < m && e - s <= kNarrow) {
         int total;
         if (e - s <= kIlp * kBfsThreads) {
-            total = level_cached(colptr, rowidx, rem, par, levelItem, s, e, cl, lds,
-                                 fr, held);
+            total = level_cached(colptr, rowidx, rem, par, levelItem, s, e, w, held);
         } else {
-            total = level_generic(colptr, rowidx, rem, par, levelItem, s, e, cl, lds);
-            held = false;
+            total = level_wide(colptr, rowidx, rem, par, levelItem, s, e, cnt, w.lds);
+            held = -1;
         }
         if (tid == 0) levelPtr[nl + 1] = e + total;
         nl++;
@@ -388,7 +491,7 @@ k_bfs(const int *__restrict__ colptr, const int *__restrict__ rowidx, int m,
       int *rem, int *par, int *cnt, int *levelItem, int *levelPtr,
       int *blocksum, BfsCtl *ctl) {
     cg::grid_group g = cg::this_grid();
-    __shared__ int lds[16];
+    __shared__ int lds[kScan];
     const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
     const int gsz = gridDim.x * blockDim.x;
 
@@ -424,20 +527,17 @@ k_bfs(const int *__restrict__ colptr, const int *__restrict__ rowidx, int m,
             // narrow frontier: workgroup 0 walks consecutive narrow levels
             // with workgroup barriers only; the rest wait at the grid sync
             if (blockIdx.x == 0)
-                bfs_narrow(colptr, rowidx, m, rem, par, levelItem, levelPtr,
-                           ctl, lds);
+                bfs_narrow(colptr, rowidx, m, rem, par, cnt, levelItem, levelPtr, ctl);
             g.sync();
             continue;
         }
         // A: decrement dependants, raise their parent position
-        for (int p = s + gtid; p < e; p += gsz) {
-            const int u = levelItem[p];
-            for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-                const int v = rowidx[q];
-                if (v == u) continue;
-                atomicSub(&rem[v], 1);
-                atomicMax(&par[v], p);
-            }
+        // (uniform trip counts in every phase: whole waves)
+        for (int base = s + blockIdx.x * blockDim.x; base < e; base += gsz) {
+            const int p = base + threadIdx.x;
+            const int u = p < e ? levelItem[p] : -1;
+            each_release<kDev>(rowidx, rem, par, u >= 0 ? colptr[u] : 0,
+                              u >= 0 ? colptr[u + 1] : 0, u, p);
         }
         g.sync();
         // B: count the children each frontier node discovers
@@ -446,32 +546,23 @@ k_bfs(const int *__restrict__ colptr, const int *__restrict__ rowidx, int m,
             const int chunk = (len + G - 1) / G;
             const int b0 = blockIdx.x * chunk;
             const int b1 = min(len, b0 + chunk);
-            for (int i = b0 + threadIdx.x; i < b1; i += blockDim.x) {
-                const int p = s + i;
-                const int u = levelItem[p];
-                int c = 0;
-                for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-                    const int v = rowidx[q];
-                    if (v != u && ld_relaxed(&rem[v]) == 0 &&
-                        ld_relaxed(&par[v]) == p)
-                        c++;
-                }
-                cnt[i] = c;
+            for (int base = b0; base < b1; base += blockDim.x) {
+                const int i = base + threadIdx.x;
+                const int u = i < b1 ? levelItem[s + i] : -1;
+                const int c = each_children<kDev>(rowidx, rem, par, u >= 0 ? colptr[u] : 0,
+                                             u >= 0 ? colptr[u + 1] : 0, u, s + i, 0, kCount);
+                if (i < b1) cnt[i] = c;
             }
         }
         g.sync();
         const int total = grid_excl_scan(g, cnt, len, blocksum, lds);
         // C: emit children in column order
-        for (int i = gtid; i < len; i += gsz) {
-            const int p = s + i;
-            const int u = levelItem[p];
-            int o = e + cnt[i];
-            for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-                const int v = rowidx[q];
-                if (v != u && ld_relaxed(&rem[v]) == 0 &&
-                    ld_relaxed(&par[v]) == p)
-                    levelItem[o++] = v;
-            }
+        for (int base = blockIdx.x * blockDim.x; base < len; base += gsz) {
+            const int i = base + threadIdx.x;
+            const int u = i < len ? levelItem[s + i] : -1;
+            each_children<kDev>(rowidx, rem, par, u >= 0 ? colptr[u] : 0,
+                           u >= 0 ? colptr[u + 1] : 0, u, s + i, i < len ? e + cnt[i] : e,
+                           [&](int at, int v) { levelItem[at] = v; });
         }
         if (gtid == 0) {
             const int nl = ctl->nlevel;
@@ -483,58 +574,6 @@ k_bfs(const int *__restrict__ colptr, const int *__restrict__ rowidx, int m,
         }
         g.sync();
     }
-}
-
-// One level [s, e) of any width inside one workgroup: the A / B / scan /
-// C phases of the narrow levels, with the counts in device memory (cnt,
-// indexed by frontier position) and a scan in chunks of the workgroup's
-// width.  A thread handles the same positions in B and C, so it reads back
-// only its own counts.
-__device__ int level_wide(const int *__restrict__ colptr,
-                          const int *__restrict__ rowidx, int *rem, int *par,
-                          int *levelItem, int s, int e, int *cnt, int *lds) {
-    const int tid = threadIdx.x;
-    for (int p = s + tid; p < e; p += blockDim.x) {
-        const int u = ld_wg(&levelItem[p]);
-        for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-            const int v = rowidx[q];
-            if (v == u) continue;
-            __hip_atomic_fetch_add(&rem[v], -1, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-            __hip_atomic_fetch_max(&par[v], p, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-    __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    int carry = 0;
-    for (int base = s; base < e; base += blockDim.x) {  // uniform trip count
-        const int p = base + tid;
-        int c = 0;
-        if (p < e) {
-            const int u = ld_wg(&levelItem[p]);
-            for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-                const int v = rowidx[q];
-                if (v != u && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p) c++;
-            }
-        }
-        int tot = 0;
-        const int off = block_excl_scan(c, lds, &tot);
-        if (p < e) cnt[p] = carry + off;
-        carry += tot;
-    }
-    for (int p = s + tid; p < e; p += blockDim.x) {
-        const int u = ld_wg(&levelItem[p]);
-        int o = e + cnt[p];
-        for (int q = colptr[u]; q < colptr[u + 1]; q++) {
-            const int v = rowidx[q];
-            if (v != u && ld_wg(&rem[v]) == 0 && ld_wg(&par[v]) == p)
-                __hip_atomic_store(&levelItem[o++], v, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_WORKGROUP);
-        }
-    }
-    return carry;
 }
 
 // The level analysis of every triangular block at once, one workgroup per
@@ -554,9 +593,7 @@ k_bfs_blocks(const int *__restrict__ colptr, const int *__restrict__ rowidx,
              const int *__restrict__ bms, const int *__restrict__ lvbase,
              int *item, int *lvptr, int *nlv, int *rem, int *par, int *cnt,
              int *stalled) {
-    __shared__ int lds[16];
-    __shared__ int cl[kNarrow];
-    __shared__ Front fr;
+    __shared__ Walk w;
     const int t = blockIdx.x, tid = threadIdx.x;
     const int up = ups[t], bm = bms[t];
     int *lp = lvptr + lvbase[t];
@@ -568,6 +605,7 @@ k_bfs_blocks(const int *__restrict__ colptr, const int *__restrict__ rowidx,
         return;
     }
     int *it = item + up;
+    if (tid == 0) w.nlong = 0;
     for (int i = tid; i < bm; i += blockDim.x) {
         rem[up + i] = rowcnt[up + i] - 1;
         par[up + i] = -1;
@@ -581,7 +619,7 @@ k_bfs_blocks(const int *__restrict__ colptr, const int *__restrict__ rowidx,
         const int i = base + tid;
         const int f = i < bm && ld_wg(&rem[up + i]) == 0 ? 1 : 0;
         int tot = 0;
-        const int off = block_excl_scan(f, lds, &tot);
+        const int off = block_excl_scan(f, w.lds, &tot);
         if (f)
             __hip_atomic_store(&it[e + off], up + i, __ATOMIC_RELAXED,
                                __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -596,17 +634,15 @@ k_bfs_blocks(const int *__restrict__ colptr, const int *__restrict__ rowidx,
     }
     int s = 0, nl = 1;
     bool bad = e == 0;
-    bool held = false;  // the level's frontier is in fr
+    int held = -1;  // which of w.fr holds the level's frontier, -1: neither
     while (e < bm && !bad) {
         const int len = e - s;
         int total;
         if (len <= kIlp * kBfsThreads) {
-            total = level_cached(colptr, rowidx, rem, par, it, s, e, cl, lds, fr, held);
+            total = level_cached(colptr, rowidx, rem, par, it, s, e, w, held);
         } else {
-            total = len <= kNarrow
-                        ? level_generic(colptr, rowidx, rem, par, it, s, e, cl, lds)
-                        : level_wide(colptr, rowidx, rem, par, it, s, e, cnt + up, lds);
-            held = false;
+            total = level_wide(colptr, rowidx, rem, par, it, s, e, cnt + up, w.lds);
+            held = -1;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();

@@ -183,8 +183,55 @@ __global__ void k_gather_csr(const int *__restrict__ order,
     }
 }
 
+// The entries of a permuted row, block by block: f(row, k, column, b, i, last)
+// for entry k, the i-th of its run in block b (a sorted row holds a block's
+// entries one after another; of several calls with last for a run, the last
+// has its last entry).  Called by whole waves; a row of more than kWideRow entries is
+// taken by its wave (a thread alone, 21,527 power-law rows, the longest of
+// 508: 275 us to count, 347 to fill, 88 and 102 like this).
+constexpr int kWideRow = 32;
+template <class F>
+__device__ inline void each_run(Geom g, const int *__restrict__ rptr,
+                                const int *__restrict__ ccol, int r, F f) {
+    const int a = r < g.m ? rptr[r] : 0, e = r < g.m ? rptr[r + 1] : 0;
+    const bool wide = e - a > kWideRow;
+    if (!wide)
+        for (int q = a, cur = -1, from = 0; q < e; q++) {
+            const int c = ccol[q];
+            if (c == r) continue;
+            const int b = block_of(g, r, c);
+            if (b != cur) {
+                cur = b;
+                from = q;
+            }
+            f(r, q, c, b, q - from, true);
+        }
+    const int lane = threadIdx.x & 63;
+    for (unsigned long long todo = __ballot(wide); todo; todo &= todo - 1) {
+        const int l = __ffsll(todo) - 1;
+        const int la = __shfl(a, l, 64), le = __shfl(e, l, 64), lr = __shfl(r, l, 64);
+        int cur = -1, from = 0;  // of the entry before
+        for (int q0 = la; q0 < le; q0 += 64) {
+            const int q = q0 + lane;
+            const int c = q < le ? ccol[q] : lr;
+            const bool off = c != lr;
+            const int b = off ? block_of(g, lr, c) : -1;
+            int before = __shfl_up(b, 1, 64);
+            if (lane == 0) before = cur;
+            const unsigned long long heads = __ballot(off && b != before);
+            const unsigned long long mine = heads & (~0ull >> (63 - lane));
+            const int start = mine ? q0 + 63 - __clzll(mine) : from;
+            // (the next lane goes on with the run)
+            const unsigned long long same = __ballot(off) & ~heads;
+            if (off) f(lr, q, c, b, q - start, lane == 63 || !(same >> (lane + 1) & 1));
+            cur = __shfl(b, 63, 64);
+            from = __shfl(start, 63, 64);
+        }
+    }
+}
+
 // Count pass over permuted rows: runs of equal block index along a sorted
-// row become one slot count; the diagonal becomes invd.
+// row become one slot count (cnt is zero before); the diagonal becomes invd.
 __global__ void k_slot_count(Geom g, const DevBlock *__restrict__ blk,
                              const int *__restrict__ bm,
                              const int *__restrict__ rptr,
@@ -192,24 +239,15 @@ __global__ void k_slot_count(Geom g, const DevBlock *__restrict__ blk,
                              const double *__restrict__ cval, int *cnt,
                              double *invd) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= g.m) return;
-    int cur = -1, run = 0;
-    for (int q = rptr[r]; q < rptr[r + 1]; q++) {
-        const int c = ccol[q];
-        if (c == r) {
-            invd[r] = 1.0 / cval[q];
-            continue;
-        }
-        const int b = block_of(g, r, c);
-        if (r - blk[b].up < 0 || r - blk[b].up >= bm[b]) continue;  // guard
-        if (b != cur) {
-            if (cur >= 0) cnt[blk[cur].slot_base + (r - blk[cur].up)] = run;
-            cur = b;
-            run = 0;
-        }
-        run++;
+    if (r < g.m) {
+        const int a = rptr[r], e = rptr[r + 1];  // (the diagonal ends a row)
+        invd[r] = 1.0 / cval[ccol[a] == r ? a : e - 1];
     }
-    if (cur >= 0) cnt[blk[cur].slot_base + (r - blk[cur].up)] = run;
+    each_run(g, rptr, ccol, r, [&](int row, int, int, int b, int i, bool last) {
+        const int at = row - blk[b].up;
+        if (at < 0 || at >= bm[b]) return;  // guard
+        if (last) cnt[blk[b].slot_base + at] = i + 1;
+    });
 }
 
 __global__ void k_slot_fill(Geom g, const DevBlock *__restrict__ blk,
@@ -220,21 +258,13 @@ __global__ void k_slot_fill(Geom g, const DevBlock *__restrict__ blk,
                             const int *__restrict__ rowptr, int *col,
                             double *val) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= g.m) return;
-    int cur = -1, o = 0;
-    for (int q = rptr[r]; q < rptr[r + 1]; q++) {
-        const int c = ccol[q];
-        if (c == r) continue;
-        const int b = block_of(g, r, c);
-        if (r - blk[b].up < 0 || r - blk[b].up >= bm[b]) continue;  // guard
-        if (b != cur) {
-            cur = b;
-            o = rowptr[blk[b].slot_base + (r - blk[b].up)];
-        }
+    each_run(g, rptr, ccol, r, [&](int row, int q, int c, int b, int i, bool) {
+        const int at = row - blk[b].up;
+        if (at < 0 || at >= bm[b]) return;  // guard
+        const int o = rowptr[blk[b].slot_base + at] + i;
         col[o] = c - blk[b].left;
         val[o] = cval[q];
-        o++;
-    }
+    });
 }
 
 // One workgroup per block: nnz and cal_longrow statistics over its slots.
@@ -458,7 +488,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     };
     // released at the end; one chunk holds the temporaries below (about 17
     // ints per row and 8 ints + 1 double per entry)
-    Arena tmp(68 * (size_t)m + 32 * (size_t)nnz + (1 << 20));
+    Arena tmp(68 * (size_t)m + 48 * (size_t)nnz + (1 << 20));
     struct Guard {
         Arena &a;
         ~Guard() { a.release(); }
@@ -539,7 +569,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         RB_HIP(hipGetLastError());
     }
     RB_HIP(hipMemsetAsync(pcolcnt + m, 0, sizeof(int), s));
-    RB_TRY(exclusive_scan_i32(pcolcnt, p->d_pcolptr, m + 1, s));
+    RB_TRY(exclusive_scan_i32(pcolcnt, p->d_pcolptr, m + 1, s, tmp));
     if (m > 0) {
         k_pcolcopy<<<nblk((long)m * 64), kT, 0, s>>>(
             d_colptr, d_rowidx, d_val, p->d_levelItem, newpos, p->d_pcolptr,
@@ -562,7 +592,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         k_iota<<<nblk(nnz), kT, 0, s>>>(iota, nnz);
         RB_HIP(hipGetLastError());
         RB_TRY(sort_pairs_i32(p->d_prowidx, sorted_rows, iota, order, nnz,
-                              bits_for(m), s));
+                              bits_for(m), s, tmp));
         k_gather_csr<<<nblk(nnz), kT, 0, s>>>(order, ecol, p->d_pval, nnz,
                                               ccol, cval);
     }
@@ -570,7 +600,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     if (nnz > 0)
         k_histogram<<<nblk(nnz), kT, 0, s>>>(p->d_prowidx, nnz, prowcnt);
     RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(prowcnt, prptr, m + 1, s));
+    RB_TRY(exclusive_scan_i32(prowcnt, prptr, m + 1, s, tmp));
 
     mark("csr");
     // ---- 9, begun here: the fused schedule's host passes need only the
@@ -635,7 +665,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         k_slot_count<<<nblk(m), kT, 0, s>>>(g, d_blk, d_bm, prptr, ccol, cval, cnt,
                                             p->d_invd);
     RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(cnt, p->d_rowptr, NS + 1, s));
+    RB_TRY(exclusive_scan_i32(cnt, p->d_rowptr, NS + 1, s, tmp));
     const int offnnz = nnz - m;  // off-diagonal entries
     RB_TRY(A.alloc(&p->d_col, offnnz));
     RB_TRY(A.alloc(&p->d_val, offnnz));
@@ -685,8 +715,8 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         }
         RB_HIP(hipMemsetAsync(fd + NS, 0, sizeof(int), s));
         RB_HIP(hipMemsetAsync(fl + NS, 0, sizeof(int), s));
-        RB_TRY(exclusive_scan_i32(fd, pd, NS + 1, s));
-        RB_TRY(exclusive_scan_i32(fl, pl, NS + 1, s));
+        RB_TRY(exclusive_scan_i32(fd, pd, NS + 1, s, tmp));
+        RB_TRY(exclusive_scan_i32(fl, pl, NS + 1, s, tmp));
         std::vector<int> hpd, hpl;
         RB_TRY(d2h(hpd, pd, (size_t)NS + 1, s));
         RB_TRY(d2h(hpl, pl, (size_t)NS + 1, s));
@@ -726,7 +756,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
             RB_HIP(hipGetLastError());
         }
         RB_HIP(hipMemsetAsync(dcnt + m, 0, sizeof(int), s));
-        RB_TRY(exclusive_scan_i32(dcnt, dptr, m + 1, s));
+        RB_TRY(exclusive_scan_i32(dcnt, dptr, m + 1, s, tmp));
         // per-triangular-block bases
         std::vector<int> tri_up(ntri), tri_m(ntri), tri_lvbase(ntri),
             tri_sb(ntri);
@@ -871,7 +901,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         RB_HIP(hipMemsetAsync(olen + m, 0, sizeof(int), s));
         k_orig_len<<<nblk(m), kT, 0, s>>>(prptr, p->d_levelItem, m, olen);
         RB_HIP(hipGetLastError());
-        RB_TRY(exclusive_scan_i32(olen, p->d_rptr, m + 1, s));
+        RB_TRY(exclusive_scan_i32(olen, p->d_rptr, m + 1, s, tmp));
         k_orig_rows<<<nblk(m), kT, 0, s>>>(prptr, ccol, cval, p->d_levelItem, m,
                                            p->d_rptr, p->d_rcol, p->d_rval);
         RB_HIP(hipGetLastError());

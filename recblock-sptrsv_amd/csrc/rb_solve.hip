@@ -847,18 +847,30 @@ static void launch_blocks(rb_plan *p, const T *val, const T *invd, T *bperm,
         launch_block<T>(p, i, val, invd, bperm, xperm, tickets, ncol, ld, nc, s);
 }
 
+int walk_launches(const rb_plan *p) {
+    int n = 0;
+    for (const Block &B : p->blocks)
+        n += B.blk_m == 0 || B.method < 0                              ? 0
+             : B.kind == 0 && B.method == 2 && B.kern == kTriRef ? B.nlv
+                                                                 : 1;
+    return n;
+}
+
 // Capture the walk on a grid of ncol columns (a power of two) into a
 // graph, once per value type and width; a replay solves the first
 // *d_ncol columns, which the prologue sets.  The scratch the graphs hold
 // grows by powers of two (at most log2 of the column cap times), so a
 // stream of solves of varying widths replays at most six graphs per type.
-// Returns false when capture is not possible; the walk is then launched
-// kernel by kernel.
+// Returns false when capture is not possible or the walk is three launches
+// at most; it is then launched kernel by kernel.  (The stream to capture on
+// alone takes 0.65 ms to create, and a replay of so few is no faster: power-
+// law factors of 3,000 and 21,527 rows in three blocks, 172 and 225 us
+// replayed, 168 and 214 launched; in seven, 166 and 253 against 168 and 257.)
 template <class T>
 static bool capture_blocks(rb_plan *p, int ncol, void **exec) {
     constexpr int ty = sizeof(T) == 8 ? 0 : 1;
     *exec = nullptr;
-    if (p->graph_failed) return false;
+    if (p->graph_failed || walk_launches(p) <= 3) return false;
     for (auto &e : p->graphs[ty])
         if (e.first == ncol) {
             *exec = e.second;
