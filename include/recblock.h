@@ -48,9 +48,11 @@ typedef enum {
                                 order: TRSV, SpMV, TRSV, ... */
 #define RB_SCHED_FUSED 2     /* one persistent dataflow launch per solve; for
                                 RB_SCHED_AUTO also the level schedule (one
-                                workgroup per factor and right-hand side),
-                                which the tuner picks for deep, narrow
-                                factors and which has no rb_plan_trace */
+                                workgroup per factor and right-hand side,
+                                for deep, narrow factors) and the flow
+                                schedule (rows in level order over all
+                                compute units, for wide levels), which the
+                                tuner picks and which have no rb_plan_trace */
 
 typedef struct {
     int schedule;      /* RB_SCHED_* */

@@ -52,7 +52,7 @@ static int lv_auto(int m, int device_id) {
 // otherwise its first timed solve settles the choice when it is more than
 // twice the fused time (its other two are then not run).
 static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
-    if (p->want_schedule == RB_SCHED_BLOCKED || (!p->fused && !p->level)) {
+    if (p->want_schedule == RB_SCHED_BLOCKED || (!p->fused && !p->level && !p->flow)) {
         p->schedule = RB_SCHED_BLOCKED;
         return tune_blocks(p, block_mode, s);
     }
@@ -75,14 +75,15 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     (void)hipEventCreate(&e1);
     // the work of a solve does not depend on the values: b = 0
     if (hipMemsetAsync(db, 0, bytes, s) != hipSuccess) st = RB_ERR_HIP;
-    enum { kBlocked, kFused, kLevel };
+    enum { kBlocked, kFused, kLevel, kFlow };
     auto timed = [&](int c, int reps) {
         float t = 0.f;
         (void)hipEventRecord(e0, s);
         for (int r = 0; r < reps && st == RB_OK; r++)
             st = c == kBlocked ? solve_blocked(p, db, m, dx, m, k, s)
                  : c == kFused ? solve_fused(p, db, m, dx, m, k, s)
-                               : solve_level(p, db, m, dx, m, k, s);
+                 : c == kLevel ? solve_level(p, db, m, dx, m, k, s)
+                               : solve_flow(p, db, m, dx, m, k, s);
         (void)hipEventRecord(e1, s);
         (void)hipEventSynchronize(e1);
         (void)hipEventElapsedTime(&t, e0, e1);
@@ -101,11 +102,12 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
         }
         return d != 0;
     };
-    double ms[3] = {0.0, 0.0, 0.0}, best = 0.0;
+    double ms[4] = {0.0, 0.0, 0.0, 0.0}, best = 0.0;
     int pick = -1;
     bool cut = false;
-    for (int c : {kLevel, kFused}) {
-        if (st != RB_OK || (c == kLevel ? !p->level : !p->fused)) continue;
+    for (int c : {kLevel, kFused, kFlow}) {
+        if (st != RB_OK || (c == kLevel ? !p->level : c == kFused ? !p->fused : !p->flow))
+            continue;
         (void)timed(c, 1);  // warm
         ms[c] = timed(c, 3) / 3.0;
         if (!tripped() && (pick < 0 || ms[c] < best)) {
@@ -133,11 +135,15 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     (void)hipFree(dx);
     if (st != RB_OK) return st;
     p->tune_ms_blocked = ms[kBlocked];
-    p->tune_ms_fused = pick == kLevel || ms[kFused] == 0.0 ? ms[kLevel] : ms[kFused];
+    p->tune_ms_fused = ms[kFused];
+    for (int c : {kLevel, kFlow})
+        if (ms[c] > 0.0 && (pick == c || p->tune_ms_fused == 0.0)) p->tune_ms_fused = ms[c];
     p->use_level = pick == kLevel;
-    p->schedule = pick == kLevel || pick == kFused ? RB_SCHED_FUSED : RB_SCHED_BLOCKED;
-    if (p->use_level) fused_destroy(p);
-    else level_destroy(p);
+    p->use_flow = pick == kFlow;
+    p->schedule = pick > kBlocked ? RB_SCHED_FUSED : RB_SCHED_BLOCKED;
+    if (p->use_level || p->use_flow) fused_destroy(p);
+    if (!p->use_level) level_destroy(p);
+    if (!p->use_flow) flow_destroy(p);
     return RB_OK;
 }
 
@@ -254,6 +260,7 @@ rb_status rb::plan_create(const int *d_colptr, const int *d_rowidx, const double
         destroy_graph(p);
         fused_destroy(p);
     level_destroy(p);
+    flow_destroy(p);
         p->arena.release();
         delete p;
         return st;
@@ -275,7 +282,9 @@ rb_status rb_solve(rb_plan *p, const double *d_b, int ldb, double *d_x,
     if (nrhs == 0) return ok();
     p->mark_first = true;
     rowcap_for_call(p, (hipStream_t)stream);
-    rb_status st = p->use_level
+    rb_status st = p->use_flow
+                       ? solve_flow(p, d_b, ldb, d_x, ldx, nrhs, (hipStream_t)stream)
+                   : p->use_level
                        ? solve_level(p, d_b, ldb, d_x, ldx, nrhs, (hipStream_t)stream)
                    : p->schedule == RB_SCHED_FUSED
                        ? solve_fused(p, d_b, ldb, d_x, ldx, nrhs,
@@ -375,6 +384,7 @@ rb_status rb_plan_destroy(rb_plan *p) {
     destroy_graph(p);
     fused_destroy(p);
     level_destroy(p);
+    flow_destroy(p);
     free_solve_scratch(p);
     p->arena.release();
     delete p;
@@ -409,7 +419,7 @@ rb_status rb_plan_info_get(const rb_plan *p, rb_plan_info *info) {
     info->nlevel = p->nlevel;
     info->schedule = p->schedule;
     info->preprocess_ms = p->preprocess_ms;
-    info->device_bytes = p->arena.bytes + level_bytes(p);
+    info->device_bytes = p->arena.bytes + level_bytes(p) + flow_bytes(p);
     for (int i = 0; i < 4; i++) info->phase_ms[i] = p->phase_ms[i];
     info->tune_ms[0] = p->tune_ms_blocked;
     info->tune_ms[1] = p->tune_ms_fused;

@@ -146,6 +146,7 @@ constexpr int kGroupSlack = 2;   // kTriGroup: rounds a wave may run ahead
 
 struct FusedPlan;
 struct LevelPlan;
+struct FlowPlan;
 
 }  // namespace rb
 
@@ -209,6 +210,10 @@ struct rb_plan {
     const int *d_partoff = nullptr;  // first row of each part
     const int *h_partoff = nullptr;  // the same on the host (while building)
     const int *d_partcap = nullptr;  // columns of each part (during a batch call)
+
+    // flow schedule (rb_flow.hip), likewise
+    rb::FlowPlan *flow = nullptr;
+    bool use_flow = false;
 
     // fused schedule (built when requested or for the tuner)
     rb::FusedPlan *fused = nullptr;
@@ -296,6 +301,9 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
 rb_status level_narrow(const rb_plan *p, hipStream_t s, bool *narrow);
 // is the level schedule estimated below the least the fused one takes?
 bool level_beats_chain(const rb_plan *p);
+// ... and below half of what any schedule takes that goes through memory
+// for every level?
+bool level_beats_walk(const rb_plan *p);
 // ws: per-solve scratch (8 bytes per row and column) instead of the plan's
 rb_status solve_level(rb_plan *p, const double *d_b, int ldb, double *d_x, int ldx,
                       int nrhs, hipStream_t s, double *ws = nullptr, size_t ws_bytes = 0);
@@ -338,6 +346,15 @@ __device__ inline void each_entry(int a, int b, F f, V... v) {
         }(__shfl(v, l, 64)...);
     }
 }
+// flow schedule (rb_flow.hip); build_flow leaves p->flow null when the matrix
+// does not fit it; ws: per-solve scratch (8 bytes per row and column, twice
+// that where b and x overlap) instead of the plan's
+rb_status build_flow(rb_plan *p, const int *d_rp, const int *d_cc, const double *d_cv,
+                     hipStream_t s);
+rb_status solve_flow(rb_plan *p, const double *d_b, int ldb, double *d_x, int ldx, int nrhs,
+                     hipStream_t s, double *ws = nullptr, size_t ws_bytes = 0);
+void flow_destroy(rb_plan *p);
+size_t flow_bytes(const rb_plan *p);
 size_t level_bytes(const rb_plan *p);
 // the same solves on caller-provided per-solve buffers (ws, ws_bytes)
 // instead of the plan's: the blocked walk needs blocked_ws_bytes(p) (one

@@ -697,6 +697,10 @@ bool level_beats_chain(const rb_plan *p) {
     return p->level && p->level->nparts == 1 && level_us(p, p->level->nsteps) < chain_us(p);
 }
 
+bool level_beats_walk(const rb_plan *p) {
+    return p->level && (p->level->nparts > 1 || level_us(p, p->level->nsteps) < 0.45 * p->nlevel);
+}
+
 rb_status level_narrow(const rb_plan *p, hipStream_t s, bool *narrow) {
     *narrow = false;
     if (level_us(p, p->nlevel) >= chain_us(p)) return RB_OK;

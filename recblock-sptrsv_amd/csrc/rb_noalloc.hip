@@ -72,9 +72,7 @@ extern "C" rb_status rb_solve_noalloc(rb_plan *p, const double *d_b, int ldb,
         return RB_OK;
     }
     const bool fused = p->schedule == RB_SCHED_FUSED;
-    const size_t need = p->use_level ? sizeof(double) * (size_t)p->m
-                        : fused      ? 16 * fused_slots(p)
-                                     : blocked_ws_bytes(p);
+    const size_t need = fused && p->fused ? 16 * fused_slots(p) : blocked_ws_bytes(p);
     if (need > kScratchBytes) {
         set_error(RB_ERR_INVALID_ARG,
                   "rb_solve_noalloc: the plan needs " + std::to_string(need) +
@@ -95,7 +93,8 @@ extern "C" rb_status rb_solve_noalloc(rb_plan *p, const double *d_b, int ldb,
     p->mark_first = true;
     rowcap_for_call(p, s);
     rb_status st =
-        p->use_level ? solve_level(p, d_b, ldb, d_x, ldx, nrhs, s, (double *)ws, kScratchBytes)
+        p->use_flow ? solve_flow(p, d_b, ldb, d_x, ldx, nrhs, s, (double *)ws, kScratchBytes)
+        : p->use_level ? solve_level(p, d_b, ldb, d_x, ldx, nrhs, s, (double *)ws, kScratchBytes)
         : fused ? solve_fused_ws(p, d_b, ldb, d_x, ldx, nrhs, s, (double *)ws,
                                kScratchBytes)
               : solve_blocked_ws(p, d_b, ldb, d_x, ldx, nrhs, s, ws,

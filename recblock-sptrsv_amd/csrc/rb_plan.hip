@@ -882,6 +882,12 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         if (narrow) RB_TRY(build_level(p, prptr, ccol, cval, s));
     }
     mark("level");
+    // flow schedule, for what neither of the others is made for
+    // (a mixed plan keeps the fused one, which has an FP32 form)
+    if (p->want_schedule == RB_SCHED_AUTO && (level_first || !p->fused) &&
+        !(p->mixed && p->fused) && !level_beats_walk(p))
+        RB_TRY(build_flow(p, prptr, ccol, cval, s));
+    mark("flow");
     // ---- 10. FP32 + FP64-refinement storage: FP32 copies of the slot
     // values, and the original matrix as CSR for the FP64 residuals (rows,
     // b, r and the x gathers all in the caller's order: the level-ordered
