@@ -865,12 +865,13 @@ int walk_launches(const rb_plan *p) {
 // at most; it is then launched kernel by kernel.  (The stream to capture on
 // alone takes 0.65 ms to create, and a replay of so few is no faster: power-
 // law factors of 3,000 and 21,527 rows in three blocks, 172 and 225 us
-// replayed, 168 and 214 launched; in seven, 166 and 253 against 168 and 257.)
+// replayed, 168 and 214 launched; in seven, 166 and 253 against 168 and 257.  The FP32 walks of a refinement,
+// which the host waits for each time, are replayed all the same.)
 template <class T>
 static bool capture_blocks(rb_plan *p, int ncol, void **exec) {
     constexpr int ty = sizeof(T) == 8 ? 0 : 1;
     *exec = nullptr;
-    if (p->graph_failed || walk_launches(p) <= 3) return false;
+    if (p->graph_failed || (ty == 0 && walk_launches(p) <= 3)) return false;
     for (auto &e : p->graphs[ty])
         if (e.first == ncol) {
             *exec = e.second;
