@@ -993,6 +993,8 @@ static int ring_class(int e) { return e == 0 ? 0 : (e <= 2 ? 2 : (e <= 4 ? 4 : 8
 
 static int words_for(int ndpp, int nring) { return words_of(ndpp, nring); }
 
+// the largest grid (waves) of a plan that is launched beside others
+static int small_grid(int ncu) { return std::max(1, ncu / 8); }
 static rb_status ensure_rhs(FusedPlan *F, int nr, hipStream_t s);
 static void device_shape(FusedPlan *F);
 
@@ -1057,12 +1059,17 @@ rb_status build_fused_host(rb_plan *p, const HostVec<int> &rp,
     };
     const int m = p->m;
     const bool fwd = p->subst == 0;
+    // waves: as many as the widest level fills, or as asked for; left to
+    // itself, as many as it takes to give no wave a second group of chains
+    // while its first is running (below), if that is at most `most`
+    const int most = fused_max_waves();
+    const bool free_waves = Wmax <= 0;
     if (Wmax <= 0) {
         int maxw = 1;
         for (int L = 0; L < p->nlevel; L++) maxw = std::max(maxw, lp[L + 1] - lp[L]);
-        Wmax = std::min(fused_max_waves(), (maxw + 63) / 64);
+        Wmax = std::min(most, (maxw + 63) / 64);
     }
-    Wmax = std::max(1, std::min(Wmax, fused_max_waves()));
+    Wmax = std::max(1, std::min(Wmax, most));
     auto qof = [&](int perm) { return fwd ? perm : m - 1 - perm; };
     auto pof = [&](int q) { return fwd ? q : m - 1 - q; };
     const int nlev = p->nlevel;
@@ -1093,47 +1100,70 @@ rb_status build_fused_host(rb_plan *p, const HostVec<int> &rp,
         for (auto &t : pool) t.join();
     }
     int W = 0;
-    std::vector<int> cnt;           // per wave count at current level
-    std::vector<int> stamp;
+    long nst = 0;  // steps
     std::vector<std::vector<int>> wave_rows;  // rows (q) per wave, in order
-    int rr = 0;
-    for (int L = 0; L < nlev; L++) {
-        const int a = lp[L], b = lp[L + 1];
-        const int width = b - a;
-        const long per = 64L * std::max(1, Wmax);
-        const int S = (int)((width + per - 1) / per);
-        const int cap = 64 * std::max(1, S);
-        for (int q = a; q < b; q++) {
-            int pref = par[q] >= 0 ? wave[par[q]] : -1;
-            int w = -1;
-            if (pref >= 0 && stamp[pref] == L && cnt[pref] < cap) w = pref;
-            else if (pref >= 0 && stamp[pref] != L) w = pref;
-            if (w < 0) {
-                if (W < Wmax) {
-                    w = W++;
-                    cnt.push_back(0);
-                    stamp.push_back(-1);
-                    wave_rows.emplace_back();
-                } else {
-                    for (int t = 0; t < W; t++) {
-                        const int c = (rr + t) % W;
-                        if (stamp[c] != L || cnt[c] < cap) {
-                            w = c;
-                            rr = (c + 1) % W;
-                            break;
+    // Rows to at most `most_waves` waves; with `alone` a row whose parent's
+    // wave is full goes to a new wave or the assignment is given up (false).
+    // A grid with more rows than columns, say, walks sideways: chains end in
+    // its first wave while new ones begin beside its last.  Given to the
+    // first, they make the waves wait for each other in a circle, and every
+    // step has to check the FIFO (333 x 217 backward: 132 us on 4 waves, 52
+    // on 6; 2000 x 100: 1,558 us on 2, 187 on 32).
+    auto assign = [&](int most_waves, bool alone) {
+        W = 0;
+        nst = 0;
+        wave_rows.clear();
+        std::vector<int> cnt;  // per wave count at current level
+        std::vector<int> stamp;
+        int rr = 0;
+        for (int L = 0; L < nlev; L++) {
+            const int a = lp[L], b = lp[L + 1];
+            const int width = b - a;
+            const long per = 64L * std::max(1, most_waves);
+            const int S = (int)((width + per - 1) / per);
+            const int cap = 64 * std::max(1, S);
+            for (int q = a; q < b; q++) {
+                int pref = par[q] >= 0 ? wave[par[q]] : -1;
+                int w = -1;
+                if (pref >= 0 && stamp[pref] == L && cnt[pref] < cap) w = pref;
+                else if (pref >= 0 && stamp[pref] != L) w = pref;
+                if (w < 0) {
+                    if (W < most_waves) {
+                        w = W++;
+                        cnt.push_back(0);
+                        stamp.push_back(-1);
+                        wave_rows.emplace_back();
+                    } else if (alone) {
+                        return false;
+                    } else {
+                        for (int t = 0; t < W; t++) {
+                            const int c = (rr + t) % W;
+                            if (stamp[c] != L || cnt[c] < cap) {
+                                w = c;
+                                rr = (c + 1) % W;
+                                break;
+                            }
                         }
                     }
                 }
+                if (stamp[w] != L) {
+                    stamp[w] = L;
+                    cnt[w] = 0;
+                }
+                if (cnt[w]++ % 64 == 0) nst++;
+                wave[q] = w;
+                wave_rows[w].push_back(q);
             }
-            if (stamp[w] != L) {
-                stamp[w] = L;
-                cnt[w] = 0;
-            }
-            cnt[w]++;
-            wave[q] = w;
-            wave_rows[w].push_back(q);
         }
-    }
+        return true;
+    };
+    // (a solve on fixed scratch, 1,024 bytes per step, that has room for the
+    // steps of the fewer waves keeps it)
+    const long fixed = (long)rb_noalloc_limit() / 1024, pad = block_steps(0);
+    const bool wide = free_waves && assign(most, true);
+    const bool over = wide && W > Wmax && nst + pad * W > fixed;
+    if (!wide || over) assign(Wmax, false);
+    if (over && nst > fixed) assign(most, true);
     // steps: a wave's rows of one level, 64 at a time; lane of the parent
     // when it is free
     HostVec<int> lvl((size_t)std::max(1, m));
@@ -1661,8 +1691,6 @@ static rb_status ensure_rhs(FusedPlan *F, int nr, hipStream_t s) {
 // kernel is bounded all the same.
 constexpr int kSmallStreams = 3;
 static std::atomic<int> g_small_plans{0};
-
-static int small_grid(int ncu) { return std::max(1, ncu / 8); }
 
 static void device_shape(FusedPlan *F) {
     if (F->ncu > 0) return;
