@@ -796,13 +796,14 @@ __global__ void __launch_bounds__(kTileThreads)
 }
 
 // The refinement's epilogue on the FP32 schedule: x (FP64, caller's order)
-// += the FP32 correction of every column not yet converged (done[c] == 0),
+// += (first: =) the FP32 correction of every column not yet converged
+// (done[c] == 0),
 // and every slot read goes back to the sentinel, so the buffers are ready
 // for the next correction without a pass of their own.
 __global__ void __launch_bounds__(kTileThreads)
     k_fused_epilogue_ir(const int *__restrict__ trow,
                         const unsigned short *__restrict__ tperm, long nslots,
-                        float *xq, double *x, long ldx, const int *status,
+                        float *xq, double *x, long ldx, bool first, const int *status,
                         const int *__restrict__ done,
                         const int *__restrict__ left) {
     if (left && *left == 0) return;
@@ -827,7 +828,7 @@ __global__ void __launch_bounds__(kTileThreads)
         const int i = k * kTileThreads + threadIdx.x;
         if (i < cnt) {
             const int row = trow[base + i];
-            if (row >= 0) xr[row] += (double)buf[tperm[base + i]];
+            if (row >= 0) xr[row] = (first ? 0.0 : xr[row]) + (double)buf[tperm[base + i]];
         }
     }
 }
@@ -1737,7 +1738,7 @@ template <class T>
 static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
                               int ldx, int nr, T *cur, T *nxt, T *brec,
                               hipStream_t s, const int *left = nullptr,
-                              const int *done = nullptr) {
+                              const int *done = nullptr, bool first = false) {
     FusedPlan *F = p->fused;
     constexpr bool f32 = sizeof(T) == 4;
     const size_t nslots = (size_t)F->nsteps * 64;
@@ -1772,7 +1773,7 @@ static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
     mark_end(p, s);
     if constexpr (f32)
         k_fused_epilogue_ir<<<tiles, kTileThreads, 0, s>>>(
-            F->d_trow, F->d_tperm, (long)nslots, cur, x, ldx, p->d_status, done,
+            F->d_trow, F->d_tperm, (long)nslots, cur, x, ldx, first, p->d_status, done,
             left);
     else
         k_fused_epilogue<T><<<tiles, kTileThreads, 0, s>>>(
@@ -1902,7 +1903,7 @@ static rb_status ensure32(rb_plan *p, int nr, hipStream_t s) {
 
 rb_status solve_fused32(rb_plan *p, const double *d_r, int ldr, double *d_x,
                         int ldx, int nrhs, hipStream_t s, const int *left,
-                        const int *done) {
+                        const int *done, bool first) {
     FusedPlan *F = p->fused;
     if (!F) {
         set_error(RB_ERR_INTERNAL, "fused schedule not built");
@@ -1916,7 +1917,7 @@ rb_status solve_fused32(rb_plan *p, const double *d_r, int ldr, double *d_x,
         const int nr = std::min(cap, nrhs - k0);
         const rb_status st = launch_group<float>(
             p, d_r + (size_t)k0 * ldr, ldr, d_x + (size_t)k0 * ldx, ldx, nr,
-            F->d_xq32, nullptr, F->d_brec32, s, left, done + k0);
+            F->d_xq32, nullptr, F->d_brec32, s, left, done + k0, first);
         if (st != RB_OK) {
             F->armed32 = false;  // an epilogue may not have run
             return st;

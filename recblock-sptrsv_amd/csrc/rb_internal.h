@@ -238,6 +238,8 @@ struct rb_plan {
     float *d_bperm32 = nullptr, *d_xperm32 = nullptr;
     int *d_rptr = nullptr, *d_rcol = nullptr;        // FP64 matrix for the
     double *d_rval = nullptr;                        // residual: CSR, original order
+    int2 *d_rwin = nullptr;  // columns that each block of its rows reads
+    int rwin = 0;            // the most of them, 0: too many for LDS
     // refinement scratch for kir right-hand sides (allocated on first use)
     int kir = 0;
     double *d_r = nullptr;                           // residual, FP64
@@ -309,7 +311,7 @@ rb_status solve_level(rb_plan *p, const double *d_b, int ldb, double *d_x, int l
                       int nrhs, hipStream_t s, double *ws = nullptr, size_t ws_bytes = 0);
 // one correction of the refinement, as solve_fused32
 rb_status solve_level32(rb_plan *p, const double *d_r, int ldr, double *d_x, int ldx, int nc,
-                        hipStream_t s, const int *left, const int *done);
+                        hipStream_t s, const int *left, const int *done, bool first);
 // A batch, straight from and to the factors' own columns: one workgroup per
 // (factor, column), listed by level_jobs (column << 16 | factor, or -1 for
 // none; nrhs[f] columns of factor f, at most 0x7fff).
@@ -321,6 +323,7 @@ rb_status solve_level_batch(rb_plan *p, const double *const *d_b, double *const 
 // right-hand sides one pass over the columns takes; permuted b / x scratch
 // for ncol of them
 int walk_cols(const rb_plan *p);
+rb_status residual_windows(rb_plan *p, Arena &tmp, hipStream_t s);
 int walk_launches(const rb_plan *p);  // kernels of the blocked walk
 rb_status scratch_cols(rb_plan *p, int ncol, hipStream_t s);
 void level_destroy(rb_plan *p);
@@ -375,7 +378,7 @@ rb_status solve_fused_ws(rb_plan *p, const double *d_b, int ldb, double *d_x,
 // be null)
 rb_status solve_fused32(rb_plan *p, const double *d_r, int ldr, double *d_x,
                         int ldx, int nrhs, hipStream_t s, const int *left,
-                        const int *done);
+                        const int *done, bool first);
 // events around a solve's main launches when timing is on: from the start
 // of the first (the entry point sets mark_first) to the end of the last
 inline void mark_start(rb_plan *p, hipStream_t s) {

@@ -873,7 +873,7 @@ static rb_status launch_level(rb_plan *p, const LevelArgs<T> &a, int grid, hipSt
 template <class T>
 static rb_status level_columns(rb_plan *p, const double *b, long ldb, double *x, long ldx,
                                int nc, double *sb, bool through, const int *left,
-                               const int *done, hipStream_t s) {
+                               const int *done, hipStream_t s, bool add = true) {
     const LevelPlan *L = p->level;
     const int m = p->m;
     LevelArgs<T> a = level_args<T>(p);
@@ -881,7 +881,7 @@ static rb_status level_columns(rb_plan *p, const double *b, long ldb, double *x,
     a.x = x;
     a.ldb = ldb;
     a.ldx = ldx;
-    a.add = true;
+    a.add = add;
     a.left = left;
     a.done = done;
     const dim3 pass(nblk(m), (nc + kPassCols - 1) / kPassCols);
@@ -899,7 +899,7 @@ static rb_status level_columns(rb_plan *p, const double *b, long ldb, double *x,
     }
     RB_TRY(launch_level<T>(p, a, a.nparts * nc, s));
     if (!L->direct) {
-        if (sizeof(T) == 4)
+        if (sizeof(T) == 4 && add)
             k_level_out<true><<<pass, kT, 0, s>>>(x, ldx, L->d_row, m, nc, sb, left, done);
         else
             k_level_out<false><<<pass, kT, 0, s>>>(x, ldx, L->d_row, m, nc, sb, left, done);
@@ -931,11 +931,12 @@ rb_status solve_level(rb_plan *p, const double *d_b, int ldb, double *d_x, int l
 }
 
 rb_status solve_level32(rb_plan *p, const double *d_r, int ldr, double *d_x, int ldx, int nc,
-                        hipStream_t s, const int *left, const int *done) {
+                        hipStream_t s, const int *left, const int *done, bool first) {
     if (p->m == 0) return RB_OK;
     // (r is the refinement's own: no overlap with x; nc is at most walk_cols)
     if (!p->level->direct) RB_TRY(scratch_cols(p, nc, s));
-    return level_columns<float>(p, d_r, ldr, d_x, ldx, nc, p->d_bperm, false, left, done, s);
+    return level_columns<float>(p, d_r, ldr, d_x, ldx, nc, p->d_bperm, false, left, done, s,
+                                !first);
 }
 
 bool level_batches(const rb_plan *p) { return p->use_level && p->level->direct; }

@@ -911,6 +911,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
         k_orig_rows<<<nblk(m), kT, 0, s>>>(prptr, ccol, cval, p->d_levelItem, m,
                                            p->d_rptr, p->d_rcol, p->d_rval);
         RB_HIP(hipGetLastError());
+        RB_TRY(residual_windows(p, tmp, s));
         RB_TRY(A.alloc(&p->d_bperm32, m));
         RB_TRY(A.alloc(&p->d_xperm32, m));
     }

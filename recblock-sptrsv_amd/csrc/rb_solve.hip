@@ -553,49 +553,66 @@ void launch_sq(int g, int nrows, int ncol, hipStream_t s, const int *rowptr,
 // the values), done[c] is set once the column has converged, and the
 // columns that are done skip every later pass.
 
-// r = b, x = 0, max |b|
-// x = 0, r = b and max |b| of column blockIdx.y: the maxima are folded
-// per workgroup, one atomic each (an atomic per wave on the column's one
-// word serialised: 55 us on 2.25M rows)
+// Columns of row i: all, or in a batch those of its factor (part) -- x and r
+// of the others are neither written nor read.
+struct RowCols {
+    const int *part, *cap;
+    __device__ int of(long i) const { return cap ? cap[part[i]] : 0x7fffffff; }
+};
+
+// A workgroup's maximum into a column's word: an atomic only where it would
+// change it.  Atomics on the columns' words, which share cache lines, take
+// 7 ns each, one after another (32 columns, 1,024 workgroups each: 212 us,
+// whatever else the kernel did).
+__device__ inline void raise_max(unsigned long long *at, unsigned long long v) {
+    if (__hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(at, v);
+}
+
+// max |b| of column blockIdx.y, folded per workgroup.  The first correction reads b itself and writes x (x = 0
+// and r = b as a pass of their own: 212 us of a batch of 1.3M rows x 32
+// columns, 17 us of 880,000 rows; the maxima alone 38 and 7).
 __global__ void __launch_bounds__(kT)
-    k_ir_init(const double *__restrict__ b, long ldb, double *x, long ldx,
-              double *r, int m, unsigned long long *bmax) {
+    k_ir_norm(const double *__restrict__ b, long ldb, int m, RowCols cols,
+              unsigned long long *bmax) {
     __shared__ double wmax[kT / 64];
     const int c = blockIdx.y;
     double mx = 0.0;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < m;
-         i += gridDim.x * blockDim.x) {
-        const double v = b[c * ldb + i];
-        r[(long)c * m + i] = v;
-        x[c * ldx + i] = 0.0;
-        mx = fmax(mx, fabs(v));
+    for (int i0 = blockIdx.x * kT + threadIdx.x; i0 < m; i0 += 4 * gridDim.x * kT) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const long i = i0 + (long)k * gridDim.x * kT;
+            if (i < m && c < cols.of(i)) mx = fmax(mx, fabs(b[c * ldb + i]));
+        }
     }
     mx = wave_max(mx);
     if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = mx;
     __syncthreads();
     if (threadIdx.x == 0) {
         for (int w = 1; w < kT / 64; w++) mx = fmax(mx, wmax[w]);
-        atomicMax(&bmax[c], (unsigned long long)__double_as_longlong(mx));
+        raise_max(&bmax[c], (unsigned long long)__double_as_longlong(mx));
     }
 }
 
-__global__ void k_ir_to32(const double *__restrict__ r, int m, float *r32,
+__global__ void k_ir_to32(const double *__restrict__ r, long ldr, int m, float *r32,
                           const int *__restrict__ done) {
     const int c = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (!done[c] && i < m) r32[(long)c * m + i] = (float)r[(long)c * m + i];
+    if (!done[c] && i < m) r32[(long)c * m + i] = (float)r[c * ldr + i];
 }
 
-// x += d (FP64 update with the FP32 correction)
+// x += d (FP64 update with the FP32 correction), the first time from zero
 __global__ void k_ir_update(const float *__restrict__ d, int m, double *x,
-                            long ldx, const int *__restrict__ done) {
+                            long ldx, bool first, const int *__restrict__ done) {
     const int c = blockIdx.y;
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (!done[c] && i < m) x[c * ldx + i] += (double)d[(long)c * m + i];
+    if (!done[c] && i < m)
+        x[c * ldx + i] = (first ? 0.0 : x[c * ldx + i]) + (double)d[(long)c * m + i];
 }
 
 // r = b - A x in the original ordering, FP64, over the original matrix as
-// CSR (rows, b, r and x all in the caller's order); max |r| per column.  G lanes per row (a power of two at or above the mean row
+// CSR (rows, b, r and x all in the caller's order); max |r| per column.
+// For matrices whose rows reach too far for the kernel below: G lanes per row
+// (a power of two at or above the mean row
 // length, as for the square blocks' SpMV) read the row's entries coalesced
 // and sum them in a fixed order (a thread per row was slow on the
 // power-law factor, whose rows reach 512 entries), for KC columns at once
@@ -608,7 +625,7 @@ template <int G, int KC>
 __global__ void __launch_bounds__(kT)
 k_ir_residual(const int *__restrict__ rptr, const int *__restrict__ rcol,
               const double *__restrict__ rval, int m, int ncol, const double *__restrict__ b, long ldb,
-              const double *__restrict__ x, long ldx, double *r,
+              const double *__restrict__ x, long ldx, double *r, RowCols cols,
               unsigned long long *rmax, const int *__restrict__ done) {
     const int c0 = blockIdx.y * KC;
     bool live[KC];
@@ -629,6 +646,7 @@ k_ir_residual(const int *__restrict__ rptr, const int *__restrict__ rcol,
     // their shuffles stay inside the group
     for (long i = ((long)blockIdx.x * blockDim.x + threadIdx.x) / G; i < m;
          i += rows_per_pass) {
+        const int nc = cols.of(i) - c0;
         double acc[KC];
 #pragma unroll
         for (int q = 0; q < KC; q++) acc[q] = 0.0;
@@ -637,7 +655,7 @@ k_ir_residual(const int *__restrict__ rptr, const int *__restrict__ rcol,
             const int cj = rcol[k];
 #pragma unroll
             for (int q = 0; q < KC; q++)
-                if (live[q]) acc[q] += v * x[(c0 + q) * ldx + cj];
+                if (live[q] && q < nc) acc[q] += v * x[(c0 + q) * ldx + cj];
         }
 #pragma unroll
         for (int q = 0; q < KC; q++) {
@@ -647,7 +665,7 @@ k_ir_residual(const int *__restrict__ rptr, const int *__restrict__ rcol,
         if (g == 0) {
 #pragma unroll
             for (int q = 0; q < KC; q++)
-                if (live[q]) {
+                if (live[q] && q < nc) {
                     const int c = c0 + q;
                     const double v = b[c * ldb + i] - acc[q];
                     r[(long)c * m + i] = v;
@@ -666,7 +684,7 @@ k_ir_residual(const int *__restrict__ rptr, const int *__restrict__ rcol,
     if (threadIdx.x < KC && live[threadIdx.x]) {
         double t = 0.0;
         for (int w = 0; w < kT / 64; w++) t = fmax(t, wmax[threadIdx.x][w]);
-        atomicMax(&rmax[c0 + threadIdx.x], (unsigned long long)__double_as_longlong(t));
+        raise_max(&rmax[c0 + threadIdx.x], (unsigned long long)__double_as_longlong(t));
     }
 }
 
@@ -677,7 +695,7 @@ static void launch_residual(rb_plan *p, int nc, const double *b, long ldb,
     const int grid = (int)std::min<long>(1024, nblk((long)m * G));
     k_ir_residual<G, KC><<<dim3(grid, (nc + KC - 1) / KC), kT, 0, s>>>(
         p->d_rptr, p->d_rcol, p->d_rval, m, nc, b, ldb, x,
-        ldx, p->d_r, p->d_norms + nc, p->d_irdone);
+        ldx, p->d_r, RowCols{p->d_part, p->d_partcap}, p->d_norms + nc, p->d_irdone);
 }
 
 template <int KC>
@@ -694,8 +712,132 @@ static void residual_kc(rb_plan *p, int nc, const double *b, long ldb,
     }
 }
 
+// The same with the x of a block of rows in LDS, column by column.  A row's
+// x lie on as many cache lines as it has entries, and the address unit takes
+// one line per clock: with x from LDS it only sees whole lines (1.3M banded
+// rows, 9 entries over 2,000 columns, up to 32 columns: 553 us with the
+// gathers, 147 like this; 880,000 rows of a grid, one column: 25 and 19).  A
+// thread keeps the entries of its kResPer rows in registers over the columns
+// of its group (the first kResEnt of a row, 4 or 10 by the mean; what is
+// longer is read again), the window's places two to a word.  Four rows to a
+// thread spilled (with ten entries 249 us), 256 threads were slower (167).  Bound: the bytes of b, r and x (the windows of
+// neighbouring blocks overlap) and the LDS reads, one per entry and column.
+// win[block]: first column and past the last of the block's rows.
+constexpr int kResT = 512, kResPer = 2, kResRows = kResT * kResPer, kResCols = 8;
+constexpr int kResWin = 7680;  // columns of a window at most (60 KB)
+template <int kResEnt>
+__global__ void __launch_bounds__(kResT)
+    k_ir_residual_win(const int *__restrict__ rptr, const int *__restrict__ rcol,
+                      const double *__restrict__ rval, int m, int ncol,
+                      const double *__restrict__ b, long ldb, const double *__restrict__ x,
+                      long ldx, double *r, const int2 *__restrict__ win, RowCols cols,
+                      unsigned long long *rmax, const int *__restrict__ done) {
+    extern __shared__ double xs[];
+    __shared__ unsigned long long lmax[kResCols];
+    __shared__ int widest;
+    const int c0 = blockIdx.y * kResCols, c1 = min(ncol, c0 + kResCols);
+    bool any = false;
+    for (int c = c0; c < c1; c++) any = any || !done[c];
+    if (!any) return;  // the whole workgroup
+    const int tid = threadIdx.x;
+    if (tid < kResCols) lmax[tid] = 0;
+    if (tid == 0) widest = 0;
+    __syncthreads();
+    const int lo = win[blockIdx.x].x, len = win[blockIdx.x].y - lo;
+    int a[kResPer], e[kResPer], nc[kResPer];
+    unsigned at[kResPer][kResEnt / 2];
+    double v[kResPer][kResEnt];
+    int most = 0;
+#pragma unroll
+    for (int k = 0; k < kResPer; k++) {
+        const int i = blockIdx.x * kResRows + k * kResT + tid;
+        const bool live = i < m;
+        a[k] = live ? rptr[i] : 0;
+        e[k] = live ? rptr[i + 1] : 0;
+        nc[k] = live ? min(cols.of(i), c1) : 0;
+        most = max(most, nc[k]);
+#pragma unroll
+        for (int j = 0; j < kResEnt; j += 2) {
+            // (no entry: zero times an x of the window)
+            unsigned w = 0;
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const bool in = a[k] + j + t < e[k];
+                const int q = in ? a[k] + j + t : a[k];
+                v[k][j + t] = in ? rval[q] : 0.0;
+                w |= (live ? (unsigned)(rcol[q] - lo) : 0u) << (16 * t);
+            }
+            at[k][j / 2] = w;
+        }
+    }
+    atomicMax(&widest, most);
+    for (int c = c0; c < c1; c++) {
+        if (done[c]) continue;
+        __syncthreads();
+        if (c >= widest) break;  // (the later columns alike)
+        for (int j = tid; j < len; j += kResT) xs[j] = x[c * ldx + lo + j];
+        __syncthreads();
+        double mx = 0.0;
+#pragma unroll
+        for (int k = 0; k < kResPer; k++) {
+            const int i = blockIdx.x * kResRows + k * kResT + tid;
+            double acc = 0.0;
+#pragma unroll
+            for (int j = 0; j < kResEnt; j++)
+                acc += v[k][j] * xs[at[k][j / 2] >> (16 * (j & 1)) & 0xffff];
+            for (int q = a[k] + kResEnt; q < e[k]; q++) acc += rval[q] * xs[rcol[q] - lo];
+            if (c < nc[k]) {
+                const double d = b[c * ldb + i] - acc;
+                r[(long)c * m + i] = d;
+                // fmax drops a NaN operand: a NaN residual counts as +inf,
+                // so its column never passes for converged
+                mx = fmax(mx, d == d ? fabs(d) : HUGE_VAL);
+            }
+        }
+        mx = wave_max(mx);
+        if ((tid & 63) == 0)
+            atomicMax(&lmax[c - c0], (unsigned long long)__double_as_longlong(mx));
+    }
+    __syncthreads();
+    if (tid < c1 - c0 && !done[c0 + tid]) raise_max(&rmax[c0 + tid], lmax[tid]);
+}
+
+__global__ void __launch_bounds__(kResT)
+    k_ir_window(const int *__restrict__ rptr, const int *__restrict__ rcol, int m, int2 *win,
+                int *most) {
+    __shared__ int lo, hi;
+    if (threadIdx.x == 0) {
+        lo = 0x7fffffff;
+        hi = 0;
+    }
+    __syncthreads();
+    int l = 0x7fffffff, h = 0;
+    for (int k = 0; k < kResPer; k++) {
+        const int i = blockIdx.x * kResRows + k * kResT + threadIdx.x;
+        each_entry(i < m ? rptr[i] : 0, i < m ? rptr[i + 1] : 0, [&](int q) {
+            l = min(l, rcol[q]);
+            h = max(h, rcol[q] + 1);
+        });
+    }
+    atomicMin(&lo, l);
+    atomicMax(&hi, h);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        win[blockIdx.x] = make_int2(lo, hi);
+        atomicMax(most, hi - lo);
+    }
+}
+
 static void residual(rb_plan *p, int nc, const double *b, long ldb,
                      const double *x, long ldx, hipStream_t s) {
+    if (p->rwin > 0) {
+        auto *kern = (long)p->nnz <= 4L * p->m ? k_ir_residual_win<4> : k_ir_residual_win<10>;
+        kern<<<dim3(nblk(p->m, kResRows), (nc + kResCols - 1) / kResCols), kResT,
+               sizeof(double) * p->rwin, s>>>(
+            p->d_rptr, p->d_rcol, p->d_rval, p->m, nc, b, ldb, x, ldx, p->d_r, p->d_rwin,
+            RowCols{p->d_part, p->d_partcap}, p->d_norms + nc, p->d_irdone);
+        return;
+    }
     switch (cols_per_thread(nc)) {
     case 4: residual_kc<4>(p, nc, b, ldb, x, ldx, s); break;
     case 2: residual_kc<2>(p, nc, b, ldb, x, ldx, s); break;
@@ -1236,6 +1378,21 @@ rb_status tune_blocks(rb_plan *p, int mode, hipStream_t s, double budget_ms,
     return RB_OK;
 }
 
+// the windows of the residual, if they fit (after d_rptr and d_rcol are there)
+rb_status residual_windows(rb_plan *p, Arena &tmp, hipStream_t s) {
+    const int nb = nblk(p->m, kResRows);
+    int *most, h = 0;
+    RB_TRY(tmp.alloc(&most, 1));
+    RB_TRY(p->arena.alloc(&p->d_rwin, nb));
+    RB_HIP(hipMemsetAsync(most, 0, sizeof(int), s));
+    k_ir_window<<<nb, kResT, 0, s>>>(p->d_rptr, p->d_rcol, p->m, p->d_rwin, most);
+    RB_HIP(hipGetLastError());
+    RB_HIP(hipMemcpyAsync(&h, most, sizeof(int), hipMemcpyDeviceToHost, s));
+    RB_HIP(hipStreamSynchronize(s));
+    p->rwin = h <= kResWin ? h : 0;
+    return RB_OK;
+}
+
 // Refinement scratch for ncol right-hand sides: r (FP64), r32 and d32
 // (FP32), m per column, and the per-column norms, flags, counts and
 // residuals; growing it frees the previous scratch.
@@ -1281,8 +1438,9 @@ void free_ir(rb_plan *p) {
 }
 
 // FP32 solves refined in FP64 (rb_solve_f32ir), all right-hand sides of a
-// walk at once: x = 0, r = b; repeat { d = solve32((float) r); x += d;
-// r = b - A x (FP64) } per column until max|r| <= tol * max|b| or
+// walk at once: x = 0, r = b (the first correction reads b and writes x
+// instead); repeat { d = solve32((float) r); x += d; r = b - A x (FP64) } per
+// column until max|r| <= tol * max|b| or
 // max_iter corrections.  The loop runs on the device; the host reads the
 // columns' flags after the second correction and each later one (one
 // synchronisation for the usual two corrections), or never when the
@@ -1299,8 +1457,13 @@ rb_status solve_f32ir(rb_plan *p, const double *d_b, int ldb, double *d_x,
     int it_max = 0;
     double rel_max = 0.0;
     bool bad = false;
-    std::vector<int> hdone(cap), hit(cap);
-    std::vector<double> hrel(cap);
+    // the columns' residuals, flags and counts lie together (ensure_ir): one
+    // copy brings all of them
+    const size_t state = (char *)p->d_irleft - (char *)p->d_irrel;
+    std::vector<double> host(state / sizeof(double) + 1);
+    const double *hrel = host.data();
+    const int *hdone = (const int *)((const char *)hrel + ((char *)p->d_irdone - (char *)p->d_irrel));
+    const int *hit = (const int *)((const char *)hrel + ((char *)p->d_iriters - (char *)p->d_irrel));
     for (int k0 = 0; k0 < nrhs && m > 0; k0 += cap) {
         const int nc = std::min(cap, nrhs - k0);
         const double *b = d_b + (size_t)k0 * ldb;
@@ -1309,24 +1472,27 @@ rb_status solve_f32ir(rb_plan *p, const double *d_b, int ldb, double *d_x,
         k_ir_reset<<<nblk(nc), kT, 0, s>>>(p->d_norms, p->d_irdone,
                                            p->d_iriters, p->d_irrel, nc,
                                            p->d_irleft);
-        k_ir_init<<<dim3(std::min(nblk(m), 1024), nc), kT, 0, s>>>(
-            b, ldb, x, ldx, p->d_r, m, p->d_norms);
+        k_ir_norm<<<dim3(std::min(nblk(m), std::max(64, 1024 / nc)), nc), kT, 0, s>>>(
+            b, ldb, m, RowCols{p->d_part, p->d_partcap}, p->d_norms);
         // max |b| / max |r| of column c: d_norms[c] / d_norms[nc + c]
         for (int it = 1; it <= max_iter; it++) {
             // once every column has converged the solve is skipped (the
             // walk's prologue sets the width its kernels read to zero; the
             // fused kernels return at once)
+            const bool first = it == 1;
+            const double *r = first ? b : p->d_r;
+            const int ldr = first ? ldb : m;
             if (p->use_level) {
-                RB_TRY(solve_level32(p, p->d_r, m, x, ldx, nc, s, p->d_irleft,
-                                     p->d_irdone));
+                RB_TRY(solve_level32(p, r, ldr, x, ldx, nc, s, p->d_irleft,
+                                     p->d_irdone, first));
             } else if (p->schedule == RB_SCHED_FUSED && p->fused) {
                 // rounding of r, the solve and x += d in the fused passes
-                RB_TRY(solve_fused32(p, p->d_r, m, x, ldx, nc, s, p->d_irleft,
-                                     p->d_irdone));
+                RB_TRY(solve_fused32(p, r, ldr, x, ldx, nc, s, p->d_irleft,
+                                     p->d_irdone, first));
             } else {
-                k_ir_to32<<<g2, kT, 0, s>>>(p->d_r, m, p->d_r32, p->d_irdone);
+                k_ir_to32<<<g2, kT, 0, s>>>(r, ldr, m, p->d_r32, p->d_irdone);
                 RB_TRY(walk<float>(p, nc, p->d_r32, m, p->d_d32, m, s, p->d_irleft));
-                k_ir_update<<<g2, kT, 0, s>>>(p->d_d32, m, x, ldx, p->d_irdone);
+                k_ir_update<<<g2, kT, 0, s>>>(p->d_d32, m, x, ldx, first, p->d_irdone);
             }
             residual(p, nc, b, ldb, x, ldx, s);
             k_ir_check<<<nblk(nc), kT, 0, s>>>(p->d_norms, p->d_norms + nc, nc,
@@ -1334,8 +1500,7 @@ rb_status solve_f32ir(rb_plan *p, const double *d_b, int ldb, double *d_x,
                                                p->d_irrel, it, p->d_irleft);
             RB_HIP(hipGetLastError());
             if (report && (it >= 2 || it == max_iter)) {
-                RB_HIP(hipMemcpyAsync(hdone.data(), p->d_irdone, sizeof(int) * nc,
-                                      hipMemcpyDeviceToHost, s));
+                RB_HIP(hipMemcpyAsync(host.data(), p->d_irrel, state, hipMemcpyDeviceToHost, s));
                 RB_HIP(hipStreamSynchronize(s));
                 bool all = true;
                 for (int c = 0; c < nc; c++) all = all && hdone[c];
@@ -1343,13 +1508,6 @@ rb_status solve_f32ir(rb_plan *p, const double *d_b, int ldb, double *d_x,
             }
         }
         if (report) {
-            RB_HIP(hipMemcpyAsync(hdone.data(), p->d_irdone, sizeof(int) * nc,
-                                  hipMemcpyDeviceToHost, s));
-            RB_HIP(hipMemcpyAsync(hit.data(), p->d_iriters, sizeof(int) * nc,
-                                  hipMemcpyDeviceToHost, s));
-            RB_HIP(hipMemcpyAsync(hrel.data(), p->d_irrel, sizeof(double) * nc,
-                                  hipMemcpyDeviceToHost, s));
-            RB_HIP(hipStreamSynchronize(s));
             for (int c = 0; c < nc; c++) {
                 if (!hdone[c]) bad = true;
                 it_max = std::max(it_max, hit[c]);
