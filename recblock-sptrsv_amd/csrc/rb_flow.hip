@@ -27,6 +27,9 @@
 // (300,001 rows backward, 5 columns: 160 us; column by column, an entry at a
 // time, 1,210 us).
 //
+// x is divided by the diagonal (a product with its reciprocal is no faster
+// here, and further off: 1.03e-16 of 4M rows, 5.6e-17 like this).
+//
 // Bound: the random reads.  4M rows, 16.6M entries outside the caches: 434 us
 // with every wait taken out of a copy, 556 with them; 75 us is what its
 // bytes would take in order.  On 300,001 rows the chain of levels, 2 us each.
@@ -63,7 +66,7 @@ struct FlowArgs {
     const int *col;     // position of an entry, -1: none
     const double *val;  // -a_ij
     const int *row;     // caller's row of a position
-    const double *dinv; // 1 / a_ii by position
+    const double *diag; // a_ii by position
     const double *b;
     double *x;
     long ldb, ldx;
@@ -154,7 +157,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
         const bool live = r < shape >> 16;
         const int p = st.pos + (live ? r : 0);
         const int row = a.row[p];
-        const double dv = a.dinv[p];
+        const double dv = a.diag[p];
         double acc[CP], bv[CP];
         bool bad = false;
         auto run = [&](auto ents, int rep) {
@@ -228,7 +231,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
             Xv<CP> x;
 #pragma unroll
             for (int c = 0; c < CP; c++)
-                x.v[c] = bad ? __builtin_nan("") : (bv[c] + sum[c]) * dv;
+                x.v[c] = bad ? __builtin_nan("") : (bv[c] + sum[c]) / dv;
             st_x<CP>(x, xs, (p * KC + c0) * 8);
 #pragma unroll
             for (int c = 0; c < CP; c++)
@@ -325,9 +328,8 @@ __global__ void k_fl_fill(const int *__restrict__ key, const int *__restrict__ r
                           const int *__restrict__ head, const int *__restrict__ sidx,
                           const int *__restrict__ off, RowGeom g, const int *__restrict__ rp,
                           const int *__restrict__ cc, const double *__restrict__ cv,
-                          const double *__restrict__ invd, const int *__restrict__ newpos,
-                          const int *__restrict__ lf, Step *step, int *col, double *val,
-                          int *row, double *dinv) {
+                          const int *__restrict__ newpos, const int *__restrict__ lf, Step *step,
+                          int *col, double *val, int *row, double *diag) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const bool live = i < g.m;
     int c = 0, k0 = 0, first = 0, past = 0, o64 = 0;
@@ -347,7 +349,7 @@ __global__ void k_fl_fill(const int *__restrict__ key, const int *__restrict__ r
             step[sidx[i]] = Step{i, gl | el << 8 | rows << 16, (unsigned)o64, chunks};
         }
         row[i] = lf[r];
-        dinv[i] = invd[r];
+        diag[i] = cv[g.fwd ? past : first - 1];
     }
     each_entry(
         first, past,
@@ -376,7 +378,7 @@ struct FlowPlan {
     int nsteps = 0;
     Step *d_step = nullptr;
     int *d_col = nullptr, *d_row = nullptr, *d_ctl = nullptr;
-    double *d_val = nullptr, *d_dinv = nullptr;
+    double *d_val = nullptr, *d_diag = nullptr;
     int ncu = 0;
     ~FlowPlan() { mem.release(); }
 };
@@ -427,12 +429,12 @@ rb_status build_flow(rb_plan *p, const int *d_rp, const int *d_cc, const double 
     RB_TRY(A.alloc(&F->d_col, ne));
     RB_TRY(A.alloc(&F->d_val, ne));
     RB_TRY(A.alloc(&F->d_row, m));
-    RB_TRY(A.alloc(&F->d_dinv, m));
+    RB_TRY(A.alloc(&F->d_diag, m));
     RB_TRY(A.alloc(&F->d_ctl, 2 * kCtl));
     k_fl_blank<<<nblk((long)ne), kT, 0, s>>>(F->d_col, F->d_val, (long)ne);
     k_fl_fill<<<nblk(m), kT, 0, s>>>(key, run, rend, order, head, sidx, off, g, d_rp, d_cc, d_cv,
-                                     p->d_invd, newpos, p->d_levelItem, F->d_step, F->d_col,
-                                     F->d_val, F->d_row, F->d_dinv);
+                                     newpos, p->d_levelItem, F->d_step, F->d_col, F->d_val,
+                                     F->d_row, F->d_diag);
     RB_HIP(hipGetLastError());
     int dev = 0, ncu = 0;
     RB_HIP(hipGetDevice(&dev));
@@ -449,7 +451,7 @@ static rb_status flow_columns(rb_plan *p, const double *b, long ldb, double *x, 
     const FlowPlan *F = p->flow;
     const long n = (long)p->m * CP * CL;
     k_flow_reset<<<nblk((n + 1) / 2), kT, 0, s>>>(xs, n, ctl);
-    FlowArgs a{F->d_step, F->d_col, F->d_val, F->d_row, F->d_dinv, b, x, ldb, ldx, ncol,
+    FlowArgs a{F->d_step, F->d_col, F->d_val, F->d_row, F->d_diag, b, x, ldb, ldx, ncol,
                p->m, F->nsteps, xs, ctl, p->d_status, p->spin_limit};
     const long takes = (long)F->nsteps * CL;
     const int grid = (int)std::max(
