@@ -722,14 +722,18 @@ __global__ void __launch_bounds__(kWG)
 }
 
 // b/diag into slot order and x out of it, one tile of kTile consecutive
-// slots per workgroup and one right-hand side per blockIdx.y.  Inside a tile
+// slots per workgroup and kTileCols right-hand sides per blockIdx.y.  Inside a tile
 // the slots are listed by ascending row (trow; padding lanes last, as -1),
 // tperm holds each listed row's slot offset in the tile and tinvd its
 // 1/diag.  The caller's b and x are then read and written in row order --
 // a chain's rows over consecutive steps are runs of consecutive rows on
 // stencil matrices -- and the slot-order side is a contiguous copy through
-// LDS.
-constexpr int kTile = 1024, kTileThreads = 256;
+// LDS.  A workgroup takes kTileCols columns with the tile's tables (14 bytes
+// a slot) in registers, two tiles of LDS in turn (1000^2 Laplacian, 16
+// columns: 92 and 80 us column by column, 72 and 65 like this; 4 columns
+// alike, 333 x 217 with 9 columns 77 us instead of 72).
+constexpr int kTile = 1024, kTileThreads = 256, kTilePer = kTile / kTileThreads;
+constexpr int kTileCols = 2;
 // tile offsets sort in the low 12 bits of a key and fit an unsigned short
 static_assert(kTile <= 4096 && (kTile & (kTile - 1)) == 0, "kTile");
 
@@ -741,27 +745,34 @@ __global__ void __launch_bounds__(kTileThreads)
     k_fused_prologue(const int *__restrict__ trow,
                      const unsigned short *__restrict__ tperm,
                      const T *__restrict__ tinvd, long nslots,
-                     const B *__restrict__ b, long ldb, T *brec,
+                     const B *__restrict__ b, long ldb, int ncol, T *brec,
                      const int *__restrict__ left) {
     if (left && *left == 0) return;
-    __shared__ T buf[kTile];
+    __shared__ T buf[2][kTile];
     const long base = (long)blockIdx.x * kTile;
     const int cnt = (int)min((long)kTile, nslots - base);
-    const B *br = b + blockIdx.y * ldb;
+    const int c0 = blockIdx.y * kTileCols, c1 = min(ncol, c0 + kTileCols);
+    int row[kTilePer], at[kTilePer];
+    T inv[kTilePer];
 #pragma unroll
-    for (int k = 0; k < kTile / kTileThreads; k++) {
+    for (int k = 0; k < kTilePer; k++) {
         const int i = k * kTileThreads + threadIdx.x;
-        if (i < cnt) {
-            const int row = trow[base + i];
-            buf[tperm[base + i]] = row >= 0 ? T(br[row]) * tinvd[base + i] : T(0);
-        }
+        row[k] = i < cnt ? trow[base + i] : -1;
+        at[k] = i < cnt ? tperm[base + i] : i;
+        inv[k] = i < cnt ? tinvd[base + i] : T(0);
     }
-    __syncthreads();
-    T *out = brec + blockIdx.y * nslots + base;
+    for (int c = c0; c < c1; c++) {
+        T *t = buf[c & 1];
 #pragma unroll
-    for (int k = 0; k < kTile / kTileThreads; k++) {
-        const int i = k * kTileThreads + threadIdx.x;
-        if (i < cnt) out[i] = buf[i];
+        for (int k = 0; k < kTilePer; k++)
+            t[at[k]] = row[k] >= 0 ? T(b[c * ldb + row[k]]) * inv[k] : T(0);
+        __syncthreads();
+        T *out = brec + c * nslots + base;
+#pragma unroll
+        for (int k = 0; k < kTilePer; k++) {
+            const int i = k * kTileThreads + threadIdx.x;
+            if (i < cnt) out[i] = t[i];
+        }
     }
 }
 
@@ -769,29 +780,34 @@ template <class T>
 __global__ void __launch_bounds__(kTileThreads)
     k_fused_epilogue(const int *__restrict__ trow,
                      const unsigned short *__restrict__ tperm, long nslots,
-                     const T *__restrict__ xq, T *x, long ldx,
+                     const T *__restrict__ xq, T *x, long ldx, int ncol,
                      const int *status, const int *__restrict__ left) {
     if (left && *left == 0) return;
-    __shared__ T buf[kTile];
+    __shared__ T buf[2][kTile];
     const long base = (long)blockIdx.x * kTile;
     const int cnt = (int)min((long)kTile, nslots - base);
-    const T *in = xq + blockIdx.y * nslots + base;
+    const int c0 = blockIdx.y * kTileCols, c1 = min(ncol, c0 + kTileCols);
     // after a watchdog trip every x of the plan's solves is a quiet NaN
     const bool tripped = (*status & 7) != 0;
+    int row[kTilePer], at[kTilePer];
 #pragma unroll
-    for (int k = 0; k < kTile / kTileThreads; k++) {
+    for (int k = 0; k < kTilePer; k++) {
         const int i = k * kTileThreads + threadIdx.x;
-        if (i < cnt) buf[i] = tripped ? T(__builtin_nan("")) : in[i];
+        row[k] = i < cnt ? trow[base + i] : -1;
+        at[k] = i < cnt ? tperm[base + i] : 0;
     }
-    __syncthreads();
-    T *xr = x + blockIdx.y * ldx;
+    for (int c = c0; c < c1; c++) {
+        T *t = buf[c & 1];
+        const T *in = xq + c * nslots + base;
 #pragma unroll
-    for (int k = 0; k < kTile / kTileThreads; k++) {
-        const int i = k * kTileThreads + threadIdx.x;
-        if (i < cnt) {
-            const int row = trow[base + i];
-            if (row >= 0) xr[row] = buf[tperm[base + i]];
+        for (int k = 0; k < kTilePer; k++) {
+            const int i = k * kTileThreads + threadIdx.x;
+            if (i < cnt) t[i] = tripped ? T(__builtin_nan("")) : in[i];
         }
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < kTilePer; k++)
+            if (row[k] >= 0) x[c * ldx + row[k]] = t[at[k]];
     }
 }
 
@@ -1751,8 +1767,9 @@ static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
         tinvd = F->d_tinvd;
         gval = F->d_gval;
     }
-    k_fused_prologue<T, double><<<tiles, kTileThreads, 0, s>>>(
-        F->d_trow, F->d_tperm, tinvd, (long)nslots, b, ldb, brec, left);
+    const dim3 groups(tiles.x, (unsigned)((nr + kTileCols - 1) / kTileCols));
+    k_fused_prologue<T, double><<<groups, kTileThreads, 0, s>>>(
+        F->d_trow, F->d_tperm, tinvd, (long)nslots, b, ldb, nr, brec, left);
     RB_HIP(hipGetLastError());
     FusedArgsT<T> args{F->d_step0, F->d_gent0, F->d_pub0, F->d_rec,
                        F->d_gsrc, gval, F->d_gmeta, F->d_pub, cur, nxt,
@@ -1776,8 +1793,8 @@ static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
             F->d_trow, F->d_tperm, (long)nslots, cur, x, ldx, first, p->d_status, done,
             left);
     else
-        k_fused_epilogue<T><<<tiles, kTileThreads, 0, s>>>(
-            F->d_trow, F->d_tperm, (long)nslots, cur, x, ldx, p->d_status, left);
+        k_fused_epilogue<T><<<groups, kTileThreads, 0, s>>>(
+            F->d_trow, F->d_tperm, (long)nslots, cur, x, ldx, nr, p->d_status, left);
     RB_HIP(hipGetLastError());
     return RB_OK;
 }
