@@ -290,6 +290,7 @@ template <> struct FV<float> {
 struct Shared {
     int ready;    // steps whose groups are all in the FIFO (resolver)
     int cons;     // steps consumed (consumer)
+    int staged;   // steps whose records are in LDS (k_staged)
     int abort;
 };
 
@@ -520,7 +521,9 @@ __device__ inline unsigned long long rotr64(unsigned long long x, int r) {
 // no pause at batch boundaries.  An entry whose step the FIFO cannot hold
 // yet (kQ steps beyond the consumer) waits like a pending one.  A group
 // longer than the window is summed across rounds (`carry`).
-template <class T>
+// ST (k_staged): fifo is the ring of staged b/diag, and a sum is taken off
+// its row's; an entry waits until its step is staged.
+template <bool ST, class T>
 __device__ __forceinline__ void resolve(const FusedArgsT<T> &a, int w, int r,
                                         int lane, T *fifo, T *rtmp, int *gtmp,
                                         T *ctmp, Shared &sh) {
@@ -572,7 +575,8 @@ __device__ __forceinline__ void resolve(const FusedArgsT<T> &a, int w, int r,
     unsigned spins = 0;
     while (base < e1) {
         nround++;
-        const int lim = lds_load_u(&sh.cons) + kQ;
+        const int lim = ST ? lds_load_u(&sh.staged) : lds_load_u(&sh.cons) + kQ;
+        if (ST) wg_acquire();
         const bool live = e < e1;
         const bool pend = live && FV<T>::pend(xv);
         const int key = gm >> 1, stp = gm >> kStepShift;
@@ -609,8 +613,9 @@ __device__ __forceinline__ void resolve(const FusedArgsT<T> &a, int w, int r,
                     q++;
                     l = (l + 1) & 63;
                 }
+                T *slot = fifo + (stp & (kQ - 1)) * 64 + (key & 63);
                 if (gtmp[l] & 1)  // complete: into the row's slot
-                    fifo[(stp & (kQ - 1)) * 64 + (key & 63)] = sum;
+                    *slot = ST ? *slot - sum : sum;
                 else
                     *ctmp = sum;  // the window's last group continues
             }
@@ -678,6 +683,21 @@ constexpr int occupancy_target(bool blk, bool multi) {
     return multi && blk ? 2 : 1;
 }
 
+// The consumer wave of a workgroup.
+__device__ inline int wave_of_block(int W) {
+    int w = blockIdx.x % W;
+    if (gridDim.x == (unsigned)W) {
+        // one column: workgroups go to the 8 XCDs round-robin (XCD =
+        // blockIdx mod 8), so XCD x takes the consecutive waves from
+        // x q + min(x, W mod 8), q = W / 8 (a bijection onto [0, W)): most
+        // wave-to-next-wave hand-offs stay in one XCD's L2.  Laplacian
+        // 1500^2, 24 waves: 216.2 -> 213.1 us.
+        const int b = blockIdx.x, x = b & 7, k = b >> 3, q = W >> 3, rem = W & 7;
+        w = x * q + min(x, rem) + k;
+    }
+    return w;
+}
+
 // One workgroup per (consumer wave w, right-hand side r): blockIdx.x =
 // r * W + w.  Right-hand sides share the records and nothing else.
 template <int NDPP, int NRING, bool BLK, bool MULTI, class T>
@@ -692,24 +712,13 @@ __global__ void __launch_bounds__(kWG)
     __shared__ Shared sh;
 
     if (a.left && *a.left == 0) return;  // every workgroup alike
-    int w = blockIdx.x % a.W;
+    const int w = wave_of_block(a.W);
     const int r = blockIdx.x / a.W;
-    if (gridDim.x == (unsigned)a.W) {
-        // one column: workgroups go to the 8 XCDs round-robin (XCD =
-        // blockIdx mod 8), so XCD x takes the consecutive waves from
-        // x q + min(x, W mod 8), q = W / 8 (a bijection onto [0, W)): most
-        // wave-to-next-wave hand-offs stay in one XCD's L2.  Laplacian
-        // 1500^2, 24 waves: 216.2 -> 213.1 us.
-        const int b = blockIdx.x, x = b & 7, k = b >> 3, q = a.W >> 3, rem = a.W & 7;
-        w = x * q + min(x, rem) + k;
-    }
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lane = threadIdx.x & 63;
     for (int i = threadIdx.x; i < kQ * 64; i += kWG) fifo[i] = T(0);
     if (threadIdx.x == 0) {
-        sh.ready = 0;
-        sh.cons = 0;
-        sh.abort = 0;
+        sh = Shared{};
         if constexpr (NRING > 0) xring[kR * 64] = T(0);
     }
     __syncthreads();
@@ -717,7 +726,159 @@ __global__ void __launch_bounds__(kWG)
         Consumer<NDPP, NRING, BLK, T> c(a, w, r, lane, xring, fifo, sh);
         c.run(w, r);
     } else if (wave == 1) {
-        resolve<T>(a, w, r, lane, fifo, rtmp, gtmp, &ctmp, sh);
+        resolve<false, T>(a, w, r, lane, fifo, rtmp, gtmp, &ctmp, sh);
+    }
+}
+
+// The same schedule for grids (one word a step, NDPP 1 or 2, block-checked)
+// where every workgroup has a compute unit to itself: four more waves stage
+// records and b/diag in LDS, kQ steps of them, and the resolver takes its
+// sums off the staged b/diag.  The consumer is left with two LDS reads, two
+// DPP moves, two FMAs and a store per step, and never waits for memory.
+// Bound: issue of one wave (3,000 x 64, one wave: 42 ns a step in k_fused, of
+// which the loads of b and records 4 and 5, clearing the FIFO 4, waiting for
+// memory 9; 30 here) and the hand-offs, 2.6 us each.  (Reading the next block's
+// first steps before its turn: 32 ns; 6 steps ahead instead of 4: alike.)
+constexpr int kStagers = 4;
+constexpr int kStagedWG = (2 + kStagers) * 64;
+
+// Stager g: blocks g, g + kStagers, ... of the wave's steps through registers
+// into the ring; a block's registers are loaded again as soon as they are
+// written.
+template <class T>
+__device__ __forceinline__ void stage(const FusedArgsT<T> &a, int w, int r, int g, int lane,
+                                      int4 *rs, T *bs, Shared &sh) {
+    constexpr int NB = block_steps(1);
+    static_assert(kQ == kStagers * NB, "a ring of one block per stager");
+    const int ns = a.step0[w + 1] - a.step0[w];
+    const __amdgpu_buffer_rsrc_t rec =
+        buf_rsrc(a.rec + (size_t)a.step0[w] * 64, (long)ns * 1024);
+    const __amdgpu_buffer_rsrc_t br =
+        buf_rsrc(a.brec + r * a.nslots + (size_t)a.step0[w] * 64, (long)ns * 64 * sizeof(T));
+    int4 rv[NB];
+    T bv[NB];
+    auto load = [&](int j, int s) {  // (past the end: nothing is fetched)
+        const int sc = min(s, ns);
+        rv[j] = __builtin_bit_cast(
+            int4, __builtin_amdgcn_raw_buffer_load_b128(rec, lane * 16, sc * 1024, 0));
+        bv[j] = FV<T>::load(br, lane * (int)sizeof(T), sc * 64 * (int)sizeof(T));
+    };
+#pragma unroll
+    for (int j = 0; j < NB; j++) load(j, g * NB + j);
+    // (the consumer goes on or aborts: its waits are bounded)
+    auto until = [&](auto f) {
+        while (!f()) {
+            if (lds_load_u(&sh.abort)) return false;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        return true;
+    };
+    for (int sb = g * NB; sb < ns; sb += kQ) {
+        // the block that was here is consumed
+        const bool ok = until([&] { return lds_load_u(&sh.cons) >= sb - kQ + NB; });
+        if (!ok) break;
+        wg_acquire();
+        int4 *rp = rs + (sb & (kQ - 1)) * 64 + lane;
+        T *bp = bs + (sb & (kQ - 1)) * 64 + lane;
+#pragma unroll
+        for (int j = 0; j < NB; j++) {
+            rp[j * 64] = rv[j];
+            bp[j * 64] = bv[j];
+            load(j, sb + kQ + j);
+        }
+        // in order: the block before is staged
+        if (!until([&] { return lds_load_u(&sh.staged) >= sb; })) break;
+        wg_release();
+        if (lane == 0) lds_store(&sh.staged, sb + NB);
+    }
+}
+
+template <int NDPP, class T>
+__device__ __forceinline__ void consume_staged(const FusedArgsT<T> &a, int w, int r, int lane,
+                                               const double2 *rs, const T *bs, Shared &sh) {
+    constexpr int NB = block_steps(1), kStep = 64 * (int)sizeof(T), kAhead = 4;
+    const unsigned long long t0 = a.trace ? now() : 0;
+    unsigned long long t_wait = 0;
+    const int ns = a.step0[w + 1] - a.step0[w];
+    const __amdgpu_buffer_rsrc_t xq = buf_rsrc(
+        a.xq + r * a.nslots + (size_t)a.step0[w] * 64, (long)ns * kStep);
+    const int laneB = lane * (int)sizeof(T);
+    T xprev = 0;
+    int avail = 0;  // steps staged and ready
+    bool ok = true;
+    for (int sb = 0; sb < ns && ok; sb += NB) {
+        if (avail < sb + NB) {
+            const unsigned long long tw = a.trace ? now() : 0;
+            unsigned spins = 0;
+            while ((avail = min(lds_load_u(&sh.ready), lds_load_u(&sh.staged))) < sb + NB) {
+                if (++spins > a.spin || lds_load_u(&sh.abort)) {
+                    if (lane == 0) {
+                        atomicOr(a.status, 2);
+                        lds_store(&sh.abort, 1);
+                    }
+                    ok = false;
+                    break;
+                }
+                __builtin_amdgcn_s_sleep(1);
+            }
+            wg_acquire();
+            if (a.trace) t_wait += now() - tw;
+        }
+        const double2 *rp = rs + (sb & (kQ - 1)) * 64 + lane;
+        const T *bp = bs + (sb & (kQ - 1)) * 64 + lane;
+        double2 f[NB];
+        T bv[NB];
+#pragma unroll
+        for (int j = 0; j < kAhead; j++) {
+            f[j] = rp[j * 64];
+            bv[j] = bp[j * 64];
+        }
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            if (u + kAhead < NB) {
+                f[u + kAhead] = rp[(u + kAhead) * 64];
+                bv[u + kAhead] = bp[(u + kAhead) * 64];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            const T xn = NDPP == 1 ? FV<T>::from_lower(xprev) : FV<T>::from_upper(xprev);
+            T acc = FV<T>::fma((T)f[u].x, xprev, bv[u]);
+            acc = FV<T>::fma((T)f[u].y, xn, acc);
+            xprev = acc;
+            FV<T>::template store<kSC1>(acc, xq, laneB, (sb + u) * kStep);
+        }
+        wg_release();
+        if (lane == 0) lds_store(&sh.cons, sb + NB);
+    }
+    if (lane == 0) lds_store(&sh.cons, 1 << 30);
+    if (a.trace && lane == 0 && r == 0) {
+        unsigned long long *tr = a.trace + (size_t)w * 16;
+        tr[1] = t_wait;
+        tr[2] = now() - t0;
+        tr[3] = ns;
+    }
+}
+
+template <int NDPP, class T>
+__global__ void __launch_bounds__(kStagedWG) k_staged(FusedArgsT<T> a) {
+    __shared__ int4 rs[kQ * 64];
+    __shared__ T bs[kQ * 64];
+    __shared__ T rtmp[64];
+    __shared__ int gtmp[64];
+    __shared__ T ctmp;
+    __shared__ Shared sh;
+    if (a.left && *a.left == 0) return;  // every workgroup alike
+    const int w = wave_of_block(a.W), r = blockIdx.x / a.W;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63;
+    if (threadIdx.x == 0) sh = Shared{};
+    __syncthreads();
+    if (wave == 0) {
+        __builtin_amdgcn_s_setprio(3);
+        consume_staged<NDPP, T>(a, w, r, lane, (const double2 *)rs, bs, sh);
+    } else if (wave == 1) {
+        resolve<true, T>(a, w, r, lane, bs, rtmp, gtmp, &ctmp, sh);
+    } else {
+        stage<T>(a, w, r, wave - 2, lane, rs, bs, sh);
     }
 }
 
@@ -1731,12 +1892,15 @@ FusedPlan::~FusedPlan() {
         if (q) (void)hipFree(q);
 }
 
+// other plans whose launches may be resident beside this one's
+static int others(const FusedPlan *F) {
+    return std::max(0, std::min(kSmallStreams, g_small_plans.load() - (F->small ? 1 : 0)));
+}
+
 // Right-hand sides that fit one cooperative launch (W workgroups each).
 static int rhs_per_launch(FusedPlan *F) {
     device_shape(F);
-    const int others = std::max(
-        0, std::min(kSmallStreams, g_small_plans.load() - (F->small ? 1 : 0)));
-    const int slots = F->per_cu * F->ncu - others * small_grid(F->ncu);
+    const int slots = F->per_cu * F->ncu - others(F) * small_grid(F->ncu);
     return std::max(1, std::min(64, slots / std::max(1, F->W)));
 }
 
@@ -1778,12 +1942,15 @@ static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
     void *kargs[] = {(void *)&args};
     mark_start(p, s);
     const bool ordinary = F->W * nr <= small_grid(F->ncu);
-    const void *kern = pick_kernel<T>(F, nr > 1);
-    hipError_t e =
-        ordinary
-            ? hipLaunchKernel(kern, dim3(F->W * nr), dim3(kWG), kargs, 0, s)
-            : hipLaunchCooperativeKernel(kern, dim3(F->W * nr), dim3(kWG),
-                                         kargs, 0, s);
+    // staged where a compute unit is left for each workgroup
+    const bool staged = F->blk && F->NRING == 0 && (F->NDPP == 1 || F->NDPP == 2) &&
+                        F->W * nr <= F->ncu - others(F) * small_grid(F->ncu);
+    const void *kern = !staged        ? pick_kernel<T>(F, nr > 1)
+                       : F->NDPP == 1 ? (const void *)k_staged<1, T>
+                                      : (const void *)k_staged<2, T>;
+    const dim3 grid(F->W * nr), wg(staged ? kStagedWG : kWG);
+    hipError_t e = ordinary ? hipLaunchKernel(kern, grid, wg, kargs, 0, s)
+                            : hipLaunchCooperativeKernel(kern, grid, wg, kargs, 0, s);
     if (e != hipSuccess)
         return status_of_hip(e, ordinary ? "hipLaunchKernel(k_fused)"
                                          : "hipLaunchCooperativeKernel(k_fused)");
