@@ -540,8 +540,10 @@ def main():
                      # counter runs cover one right-hand side
                      "traffic": measured_traffic(wname, sched)
                                 if args.rhs == 1 else None,
-                     "kernel": "k_fused" if sched == "fused" else
-                               "blocked block walk (graph of block kernels)",
+                     "kernel": "blocked block walk (graph of block kernels)"
+                               if sched != "fused" else
+                               "k_level or k_flow" if plan.trace() is None
+                               else "k_staged or k_fused",
                      "launch_ms": round(launch_ms, 5),
                      "algorithmic_bytes_per_launch": B,
                      "cache": "warm: repeated solves, the factor's data "
