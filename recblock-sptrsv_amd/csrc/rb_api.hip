@@ -44,13 +44,14 @@ static int lv_auto(int m, int device_id) {
 // Kernel choice per block (tune_blocks, rb_opts.block_kernels) and the
 // schedule.  BLOCKED and FUSED are taken as asked (a fused-only plan keeps
 // the reference selector's block kernels without timing them); AUTO times
-// warm solves of each candidate on scratch right-hand sides (tune_rhs
-// columns per call, default 1) and keeps the faster (the plan is built for
-// both).  The fused schedule is timed first: with one column, the block
-// kernel timing stops as soon as the timed blocks alone take more than
-// twice the fused solve, and the blocked schedule is then not timed at all;
+// warm solves of each candidate that was built (level, fused, flow, blocked)
+// on scratch right-hand sides (tune_rhs columns per call, default 1) and
+// keeps the fastest.  The blocked schedule comes last: with one column, the
+// block kernel timing stops as soon as the timed blocks alone take more than
+// twice the best of the others, and the schedule is then not timed at all;
 // otherwise its first timed solve settles the choice when it is more than
-// twice the fused time (its other two are then not run).
+// 1.5 times the best (its other two are then not run; solves of one schedule
+// differ by a few per cent).
 static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     if (p->want_schedule == RB_SCHED_BLOCKED || (!p->fused && !p->level && !p->flow)) {
         p->schedule = RB_SCHED_BLOCKED;
@@ -129,7 +130,7 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     if (st == RB_OK && !cut && !clear) {
         (void)timed(kBlocked, 1);  // warm (captures the walk)
         const double t1 = timed(kBlocked, 1);
-        ms[kBlocked] = t1 > 2.0 * best && pick >= 0 ? t1 : (t1 + timed(kBlocked, 2)) / 3.0;
+        ms[kBlocked] = t1 > 1.5 * best && pick >= 0 ? t1 : (t1 + timed(kBlocked, 2)) / 3.0;
         if (!tripped() && (pick < 0 || ms[kBlocked] <= best)) pick = kBlocked;
     }
     (void)hipEventDestroy(e0);
