@@ -305,7 +305,9 @@ rb_status rb_batch_create(int nfactors, const int *const *d_colptr,
 
 /* Factor f solves nrhs[f] right-hand sides d_b[f] (m[f] x nrhs[f],
  * leading dimension ldb[f]) into d_x[f] (ldx[f]); nrhs[f] may be 0.
- * Host arrays of device pointers.  Stream-ordered; the per-call tables are
+ * Host arrays of device pointers.  A d_x may lie over any d_b (the call then
+ * takes a copy of all of them first, unless each lies over its own, in place).
+ * Stream-ordered; the per-call tables are
  * staged through pinned memory, so the arrays may be reused on return. */
 rb_status rb_batch_solve(rb_batch *batch, const double *const *d_b,
                          const int *ldb, double *const *d_x, const int *ldx,

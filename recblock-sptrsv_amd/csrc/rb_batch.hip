@@ -13,6 +13,7 @@
 // the per-row column counts written for the call), and a scatter pass
 // copies the solutions back.
 #include <algorithm>
+#include <cstdint>
 #include <cstring>
 #include <vector>
 
@@ -112,6 +113,57 @@ using namespace rb;
 static rb_status done() {
     set_error(RB_OK, "");
     return RB_OK;
+}
+
+// Memory [lo, hi) of one b or x (a factor's columns together, or one column);
+// alone: solving b into the x at the same address reads each b before it
+// is overwritten.
+struct Span {
+    uintptr_t lo, hi;
+    int id;
+    bool alone;
+};
+
+// Does an x overlap a b other than its own in place, or another x?
+static bool spans_clash(const std::vector<Span> &bs, std::vector<Span> &xs) {
+    std::sort(xs.begin(), xs.end(), [](const Span &a, const Span &b) { return a.lo < b.lo; });
+    for (size_t i = 1; i < xs.size(); i++)
+        if (xs[i].lo < xs[i - 1].hi) return true;
+    for (const Span &b : bs) {
+        // (disjoint: ascending ends too)
+        auto x = std::partition_point(xs.begin(), xs.end(),
+                                      [&](const Span &v) { return v.hi <= b.lo; });
+        for (; x != xs.end() && x->lo < b.hi; ++x)
+            if (!(x->id == b.id && x->lo == b.lo && b.alone)) return true;
+    }
+    return false;
+}
+
+// Would a solve straight from the callers' b into their x, every (factor,
+// column) for itself and in no order, overwrite a b that is still to be read?
+// The factors' arrays as wholes first; where those overlap (row ranges of one
+// matrix do, say) column by column.
+static bool batch_overlaps(const rb_batch *B, const double *const *d_b, const int *ldb,
+                           double *const *d_x, const int *ldx, const int *nrhs) {
+    std::vector<Span> bs, xs;
+    auto span = [](const double *p, long n, int id, bool alone) {
+        return Span{(uintptr_t)p, (uintptr_t)(p + n), id, alone};
+    };
+    for (int f = 0; f < B->nf; f++) {
+        const long m = B->m[f], k = nrhs[f];
+        if (m == 0 || k == 0) continue;
+        bs.push_back(span(d_b[f], (k - 1) * ldb[f] + m, f, ldb[f] == ldx[f] || k == 1));
+        xs.push_back(span(d_x[f], (k - 1) * ldx[f] + m, f, true));
+    }
+    if (!spans_clash(bs, xs)) return false;
+    bs.clear();
+    xs.clear();
+    for (int f = 0, id = 0; f < B->nf; f++)
+        for (long c = 0; B->m[f] > 0 && c < nrhs[f]; c++, id++) {
+            bs.push_back(span(d_b[f] + c * ldb[f], B->m[f], id, true));
+            xs.push_back(span(d_x[f] + c * ldx[f], B->m[f], id, true));
+        }
+    return spans_clash(bs, xs);
 }
 
 extern "C" {
@@ -221,15 +273,11 @@ rb_status rb_batch_create(int nf, const int *const *d_colptr,
 
 rb_plan *rb_batch_plan(rb_batch *B) { return B ? B->plan : nullptr; }
 
-// Check the call's arguments and upload its tables, with the level
-// schedule's workgroups when asked for (*njobs of them).
-// Returns the most columns of a factor through *kmax.
-static rb_status batch_tables(rb_batch *B, const double *const *d_b, const int *ldb,
-                              double *const *d_x, const int *ldx, const int *nrhs,
-                              hipStream_t s, int *kmax, int *njobs) {
-    const int nf = B->nf;
+// Check a call's arguments; the most columns of a factor through *kmax.
+static rb_status batch_args(const rb_batch *B, const double *const *d_b, const int *ldb,
+                            double *const *d_x, const int *ldx, const int *nrhs, int *kmax) {
     int k = 0;
-    for (int f = 0; f < nf; f++) {
+    for (int f = 0; f < B->nf; f++) {
         if (nrhs[f] < 0 || (nrhs[f] > 0 && (!d_b[f] || !d_x[f] ||
                                             ldb[f] < B->m[f] || ldx[f] < B->m[f]))) {
             set_error(RB_ERR_INVALID_ARG, "invalid solve arguments for factor " +
@@ -238,8 +286,16 @@ static rb_status batch_tables(rb_batch *B, const double *const *d_b, const int *
         }
         k = std::max(k, nrhs[f]);
     }
-    *kmax = k;
-    if (k == 0 || B->n_total == 0) return RB_OK;
+    *kmax = B->n_total == 0 ? 0 : k;
+    return RB_OK;
+}
+
+// Upload a call's tables, with the level schedule's workgroups when asked
+// for (*njobs of them).
+static rb_status batch_tables(rb_batch *B, const double *const *d_b, const int *ldb,
+                              double *const *d_x, const int *ldx, const int *nrhs,
+                              hipStream_t s, int *njobs) {
+    const int nf = B->nf;
     std::vector<int> jobs;
     if (njobs) {
         level_jobs(B->plan, nrhs, jobs);
@@ -293,9 +349,10 @@ static rb_status batch_stage(rb_batch *B, const double *const *d_b,
                              const int *ldx, const int *nrhs, hipStream_t s,
                              int *kmax) {
     const int nf = B->nf;
-    RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, kmax, nullptr));
+    RB_TRY(batch_args(B, d_b, ldb, d_x, ldx, nrhs, kmax));
     const int k = *kmax;
-    if (k == 0 || B->n_total == 0) return RB_OK;
+    if (k == 0) return RB_OK;
+    RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, nullptr));
     if (k > B->kalloc) {
         RB_HIP(hipStreamSynchronize(s));
         if (B->d_B) RB_HIP(hipFree(B->d_B));
@@ -340,11 +397,14 @@ rb_status rb_batch_solve(rb_batch *B, const double *const *d_b,
     }
     hipStream_t s = (hipStream_t)stream;
     int k = 0;
-    int widest = 0;
-    for (int f = 0; f < B->nf; f++) widest = std::max(widest, nrhs[f]);
-    if (level_batches(B->plan) && widest <= 0x7fff) {
+    RB_TRY(batch_args(B, d_b, ldb, d_x, ldx, nrhs, &k));
+    if (k == 0) return done();
+    // straight from and to the factors' own columns, unless an x lies over a
+    // b that another workgroup reads: then by way of the union's columns
+    if (level_batches(B->plan) && k <= 0x7fff &&
+        !batch_overlaps(B, d_b, ldb, d_x, ldx, nrhs)) {
         int njobs = 0;
-        RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, &k, &njobs));
+        RB_TRY(batch_tables(B, d_b, ldb, d_x, ldx, nrhs, s, &njobs));
         if (njobs == 0) return done();
         B->plan->mark_first = true;
         RB_TRY(solve_level_batch(B->plan, B->d_bp, B->d_xp, B->d_ld, B->d_ld + B->nf,
@@ -352,7 +412,7 @@ rb_status rb_batch_solve(rb_batch *B, const double *const *d_b,
         return done();
     }
     RB_TRY(batch_stage(B, d_b, ldb, d_x, ldx, nrhs, s, &k));
-    if (k == 0 || B->n_total == 0) return done();
+    if (k == 0) return done();
     RB_TRY(rb_solve(B->plan, B->d_B, B->n_total, B->d_X, B->n_total, k, stream));
     RB_TRY(batch_unstage(B, k, s));
     return done();
@@ -372,7 +432,7 @@ rb_status rb_batch_solve_f32ir(rb_batch *B, const double *const *d_b,
     if (iters) *iters = 0;
     if (relres) *relres = 0.0;
     RB_TRY(batch_stage(B, d_b, ldb, d_x, ldx, nrhs, s, &k));
-    if (k == 0 || B->n_total == 0) return done();
+    if (k == 0) return done();
     B->plan->d_partcap = B->d_ld + 2 * B->nf;
     const rb_status st = rb_solve_f32ir(B->plan, B->d_B, B->n_total, B->d_X,
                                         B->n_total, k, tol, max_iter, stream,
