@@ -160,7 +160,12 @@ rb_status rb_plan_create(const int *d_colptr, const int *d_rowidx,
 /* Solve op(T) X = B for nrhs right-hand sides: d_b is m x nrhs
  * column-major with leading dimension ldb >= m, d_x likewise with ldx.
  * Stream-ordered and asynchronous (no host synchronisation); d_b is not
- * modified.  One plan must not run two solves at once; distinct plans may. */
+ * modified, except where d_x lies over it: a column of d_x may lie over any
+ * of d_b (in place, or some rows or columns off).  Where there are more
+ * columns than one pass takes and, with differing leading dimensions, no
+ * order of the passes reads every b before it is overwritten, the call is
+ * refused with RB_ERR_INVALID_ARG.
+ * One plan must not run two solves at once; distinct plans may. */
 rb_status rb_solve(rb_plan *plan, const double *d_b, int ldb, double *d_x,
                    int ldx, int nrhs, void *stream);
 

@@ -2,6 +2,7 @@
 // points with the reference's signatures.
 #include <chrono>
 #include <cmath>
+#include <cstdlib>
 #include <cstring>
 
 #include "rb_internal.h"
@@ -30,6 +31,29 @@ static rb_status ok() {
     g_status = RB_OK;
     g_msg.clear();
     return RB_OK;
+}
+
+rb_status column_groups(const double *b, long ldb, const double *x, long ldx, int m, int nrhs,
+                        int cap, ColumnGroups *out) {
+    out->cap = cap;
+    out->n = (nrhs + cap - 1) / cap;
+    out->down = false;
+    if (out->n < 2 || !part_overlap(b, ldb, x, ldx, m, nrhs)) return RB_OK;
+    // (columns do not overlap each other, so b's column k meets two of x at most)
+    bool up = true, down = true;
+    const long d = b - x;
+    for (long k = 0; k < nrhs; k++)
+        for (long j = std::max(0L, (d + k * ldb) / ldx - 1);
+             j < std::min((long)nrhs, (d + k * ldb) / ldx + 2); j++)
+            if (std::abs(d + k * ldb - j * ldx) < m) {
+                up = up && j / cap >= k / cap;
+                down = down && j / cap <= k / cap;
+            }
+    out->down = !up;
+    if (up || down) return RB_OK;
+    set_error(RB_ERR_INVALID_ARG,
+              "x lies over b so that no order of the columns reads each b in time");
+    return RB_ERR_INVALID_ARG;
 }
 
 static int lv_auto(int m, int device_id) {

@@ -474,7 +474,8 @@ rb_status solve_flow(rb_plan *p, const double *d_b, int ldb, double *d_x, int ld
     const size_t col = sizeof(double) * (size_t)m;
     int cap = 8;  // columns at a time
     while (cap > 1 && (long)m * cap * 8 > 0x7fffffffL) cap /= 2;
-    // b is copied first where x would overwrite what is still to be read
+    // a group's b is copied first where x would overwrite what is still to be
+    // read
     const bool copy = part_overlap(d_b, ldb, d_x, ldx, m, nrhs);
     int group = copy ? std::min(nrhs, walk_cols(p)) : nrhs;  // columns copied at a time
     double *xs = ws, *bc = nullptr;
@@ -494,7 +495,10 @@ rb_status solve_flow(rb_plan *p, const double *d_b, int ldb, double *d_x, int ld
         xs = p->d_xperm;
         bc = p->d_bperm;
     }
-    for (int g = 0; g < nrhs; g += group) {
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, m, nrhs, group, &grp));
+    for (int i = 0; i < grp.n; i++) {
+        const int g = grp.at(i);
         const int ng = std::min(group, nrhs - g);
         const double *b = d_b + (size_t)g * ldb;
         long lb = ldb;

@@ -1977,8 +1977,11 @@ rb_status solve_fused(rb_plan *p, const double *d_b, int ldb, double *d_x,
     const size_t nslots = (size_t)F->nsteps * 64;
     device_shape(F);
     const int cap = nrhs > 1 ? rhs_per_launch(F) : 1;
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, p->m, nrhs, cap, &grp));
     RB_TRY(ensure_rhs(F, std::min(nrhs, cap), s));
-    for (int k0 = 0; k0 < nrhs; k0 += cap) {
+    for (int i = 0; i < grp.n; i++) {
+        const int k0 = grp.at(i);
         const int nr = std::min(cap, nrhs - k0);
         const int cb = F->epoch & 1, nb = cb ^ 1;
         double *cur = F->d_xq + (size_t)cb * F->nr_alloc * nslots;
@@ -2024,7 +2027,10 @@ rb_status solve_fused_ws(rb_plan *p, const double *d_b, int ldb, double *d_x,
         return RB_ERR_INVALID_ARG;
     }
     const int cap = std::min(fit, nrhs > 1 ? rhs_per_launch(F) : 1);
-    for (int k0 = 0; k0 < nrhs; k0 += cap) {
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, p->m, nrhs, cap, &grp));
+    for (int i = 0; i < grp.n; i++) {
+        const int k0 = grp.at(i);
         const int nr = std::min(cap, nrhs - k0);
         double *cur = ws;
         double *brec = ws + (size_t)nr * nslots;

@@ -332,6 +332,17 @@ inline bool part_overlap(const double *b, long ldb, const double *x, long ldx, i
     if (b == x && (ldb == ldx || n == 1)) return false;
     return b < x + (n - 1) * ldx + m && x < b + (n - 1) * ldb + m;
 }
+// Groups of at most cap columns, in the order in which no group's x overwrites
+// a b that a later group reads (a group reads all of its own b first): the
+// i-th begins at column at(i).
+struct ColumnGroups {
+    int cap, n = 0;
+    bool down = false;
+    int at(int i) const { return (down ? n - 1 - i : i) * cap; }
+};
+// ... or an error where neither order is one (rb_api.hip)
+rb_status column_groups(const double *b, long ldb, const double *x, long ldx, int m, int nrhs,
+                        int cap, ColumnGroups *out);
 // Every entry [a, b) of every lane's row, f(k, v...) with v the row's values;
 // called by whole waves.  A row of more than 32 entries is taken by its wave:
 // one thread alone goes through it entry by entry (21,527 power-law rows, the

@@ -922,11 +922,15 @@ rb_status solve_level(rb_plan *p, const double *d_b, int ldb, double *d_x, int l
         set_error(RB_ERR_INVALID_ARG, "workspace too small for one column");
         return RB_ERR_INVALID_ARG;
     }
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, m, nrhs, cap, &grp));
     if (!ws) RB_TRY(scratch_cols(p, std::min(cap, nrhs), s));
-    for (int k = 0; k < nrhs; k += cap)
+    for (int i = 0; i < grp.n; i++) {
+        const int k = grp.at(i);
         RB_TRY(level_columns<double>(p, d_b + (size_t)k * ldb, ldb, d_x + (size_t)k * ldx, ldx,
                                      std::min(cap, nrhs - k), ws ? ws : p->d_bperm, through,
                                      nullptr, nullptr, s));
+    }
     return RB_OK;
 }
 

@@ -1177,9 +1177,13 @@ rb_status solve_blocked(rb_plan *p, const double *d_b, int ldb, double *d_x,
                         int ldx, int nrhs, hipStream_t s) {
     if (p->m == 0) return RB_OK;
     const int cap = walk_cols(p);
-    for (int k = 0; k < nrhs; k += cap)
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, p->m, nrhs, cap, &grp));
+    for (int i = 0; i < grp.n; i++) {
+        const int k = grp.at(i);
         RB_TRY(walk<double>(p, std::min(cap, nrhs - k), d_b + (size_t)k * ldb,
                             ldb, d_x + (size_t)k * ldx, ldx, s));
+    }
     return RB_OK;
 }
 
@@ -1199,7 +1203,10 @@ rb_status solve_blocked_ws(rb_plan *p, const double *d_b, int ldb,
     double *bperm = (double *)ws;
     double *xperm = bperm + m;
     int *tickets = (int *)(xperm + m);
-    for (int k = 0; k < nrhs; k++) {
+    ColumnGroups grp;
+    RB_TRY(column_groups(d_b, ldb, d_x, ldx, m, nrhs, 1, &grp));
+    for (int i = 0; i < grp.n; i++) {
+        const int k = grp.at(i);
         const int pro = nblk(m > p->ntri ? m : p->ntri);
         k_prologue<double><<<pro, kT, 0, s>>>(d_b + (size_t)k * ldb, ldb,
                                               p->d_levelItem, m, m, bperm,
