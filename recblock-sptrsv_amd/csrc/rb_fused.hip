@@ -51,6 +51,7 @@
 #include <vector>
 
 #include "rb_internal.h"
+#include "rb_residency.h"
 
 namespace rb {
 
@@ -1171,8 +1172,6 @@ static int ring_class(int e) { return e == 0 ? 0 : (e <= 2 ? 2 : (e <= 4 ? 4 : 8
 
 static int words_for(int ndpp, int nring) { return words_of(ndpp, nring); }
 
-// the largest grid (waves) of a plan that is launched beside others
-static int small_grid(int ncu) { return std::max(1, ncu / 8); }
 static rb_status ensure_rhs(FusedPlan *F, int nr, hipStream_t s);
 static void device_shape(FusedPlan *F);
 
@@ -1863,11 +1862,10 @@ static rb_status ensure_rhs(FusedPlan *F, int nr, hipStream_t s) {
 // ordinary).  Launches of at most ncu / 8 workgroups -- single-column solves
 // of plans with few waves -- are ordinary launches: such a grid is resident
 // once dispatched as long as the device's other resident work leaves it that
-// many workgroup slots.  The cooperative (multi-column) launches size
-// themselves to leave those slots to up to kSmallStreams other live plans
-// whose solves may be ordinary launches on other streams.  Every wait in the
-// kernel is bounded all the same.
-constexpr int kSmallStreams = 3;
+// many compute units.  The cooperative (multi-column) launches size
+// themselves to be resident beside up to kSmallStreams other live plans
+// whose solves may be ordinary launches on other streams, a compute unit for
+// each of their workgroups.  Every wait in the kernel is bounded all the same.
 static std::atomic<int> g_small_plans{0};
 
 static void device_shape(FusedPlan *F) {
@@ -1900,7 +1898,7 @@ static int others(const FusedPlan *F) {
 // Right-hand sides that fit one cooperative launch (W workgroups each).
 static int rhs_per_launch(FusedPlan *F) {
     device_shape(F);
-    const int slots = F->per_cu * F->ncu - others(F) * small_grid(F->ncu);
+    const int slots = resident_slots(F->per_cu, F->ncu, others(F));
     return std::max(1, std::min(64, slots / std::max(1, F->W)));
 }
 
@@ -1944,7 +1942,7 @@ static rb_status launch_group(rb_plan *p, const double *b, int ldb, double *x,
     const bool ordinary = F->W * nr <= small_grid(F->ncu);
     // staged where a compute unit is left for each workgroup
     const bool staged = F->blk && F->NRING == 0 && (F->NDPP == 1 || F->NDPP == 2) &&
-                        F->W * nr <= F->ncu - others(F) * small_grid(F->ncu);
+                        F->W * nr <= resident_slots(1, F->ncu, others(F));
     const void *kern = !staged        ? pick_kernel<T>(F, nr > 1)
                        : F->NDPP == 1 ? (const void *)k_staged<1, T>
                                       : (const void *)k_staged<2, T>;
