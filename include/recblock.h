@@ -46,13 +46,16 @@ typedef enum {
 #define RB_SCHED_AUTO 0      /* the library's tuner picks (default) */
 #define RB_SCHED_BLOCKED 1   /* per-block kernels in the reference selector's
                                 order: TRSV, SpMV, TRSV, ... */
-#define RB_SCHED_FUSED 2     /* one persistent dataflow launch per solve; for
-                                RB_SCHED_AUTO also the level schedule (one
-                                workgroup per factor and right-hand side,
-                                for deep, narrow factors) and the flow
-                                schedule (rows in level order over all
-                                compute units, for wide levels), which the
-                                tuner picks and which have no rb_plan_trace */
+#define RB_SCHED_FUSED 2     /* one persistent dataflow launch per solve */
+/* Two more that RB_SCHED_AUTO picks from (rb_plan_info reports them as
+ * RB_SCHED_FUSED, rb_plan_schedule as what they are; no rb_plan_trace).  Asked
+ * for by name, a factor that does not fit is refused with
+ * RB_ERR_INVALID_ARG. */
+#define RB_SCHED_LEVEL 3     /* one workgroup per factor and right-hand side,
+                                for deep, narrow factors (rows of at most 512
+                                off-diagonal entries) */
+#define RB_SCHED_FLOW 4      /* rows in level order over all compute units,
+                                for wide levels (not for batches) */
 
 typedef struct {
     int schedule;      /* RB_SCHED_* */
@@ -187,19 +190,26 @@ typedef struct {
     int m, nnz, substitution, lv;
     int nblocks;          /* 2^(lv+1) - 1 */
     int nlevel;           /* global level count */
-    int schedule;         /* schedule a solve uses (RB_SCHED_BLOCKED/FUSED) */
+    int schedule;         /* RB_SCHED_BLOCKED, or RB_SCHED_FUSED for any of
+                             the others (rb_plan_schedule) */
     double preprocess_ms; /* plan build time (phases 0-2 below) */
     size_t device_bytes;  /* device memory held by the plan */
     double phase_ms[4];   /* host-clock ms of the build's phases: level
                              analysis; reorder, partition, blocks, selector
                              and storage; fused schedule build; schedule
                              tuning (timed solves, not in preprocess_ms) */
-    double tune_ms[2];    /* warm solve time of the blocked / fused schedule
-                             at tune_rhs columns when RB_SCHED_AUTO timed
-                             both, else 0 */
+    double tune_ms[2];    /* RB_SCHED_AUTO: warm solve time at tune_rhs
+                             columns of the blocked schedule, and of the
+                             picked one of the others (where blocked was
+                             picked, of the fused or else of another that
+                             was timed); 0: not timed */
 } rb_plan_info;
 
 rb_status rb_plan_info_get(const rb_plan *plan, rb_plan_info *info);
+
+/* The schedule a solve runs (RB_SCHED_BLOCKED .. RB_SCHED_FLOW; -1 for a null
+ * plan).  No counterpart in the reference. */
+int rb_plan_schedule(const rb_plan *plan);
 
 /* Per-block selector inputs and decisions, host arrays of nblocks entries
  * (any pointer may be NULL).  Triangular blocks are even indices, square

@@ -66,7 +66,8 @@ static int lv_auto(int m, int device_id) {
 }
 
 // Kernel choice per block (tune_blocks, rb_opts.block_kernels) and the
-// schedule.  BLOCKED and FUSED are taken as asked (a fused-only plan keeps
+// schedule.  BLOCKED, FUSED, LEVEL and FLOW are taken as asked (a plan that
+// never walks its blocks keeps
 // the reference selector's block kernels without timing them); AUTO times
 // warm solves of each candidate that was built (level, fused, flow, blocked)
 // on scratch right-hand sides (tune_rhs columns per call, default 1) and
@@ -81,9 +82,12 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
         p->schedule = RB_SCHED_BLOCKED;
         return tune_blocks(p, block_mode, s);
     }
-    if (p->want_schedule == RB_SCHED_FUSED) {
+    if (p->want_schedule >= RB_SCHED_FUSED && p->want_schedule <= RB_SCHED_FLOW) {
         p->schedule = RB_SCHED_FUSED;
-        return tune_blocks(p, 1, s);
+        p->use_level = p->want_schedule == RB_SCHED_LEVEL;
+        p->use_flow = p->want_schedule == RB_SCHED_FLOW;
+        // (a mixed plan on the flow schedule refines on the blocked walk)
+        return tune_blocks(p, p->use_flow && p->mixed ? block_mode : 1, s);
     }
     const int m = p->m;
     const int k = std::max(1, std::min(p->tune_rhs, 64));
@@ -452,6 +456,13 @@ rb_status rb_plan_info_get(const rb_plan *p, rb_plan_info *info) {
     info->tune_ms[0] = p->tune_ms_blocked;
     info->tune_ms[1] = p->tune_ms_fused;
     return ok();
+}
+
+int rb_plan_schedule(const rb_plan *p) {
+    return !p            ? -1
+           : p->use_level ? RB_SCHED_LEVEL
+           : p->use_flow  ? RB_SCHED_FLOW
+                          : p->schedule;
 }
 
 rb_status rb_plan_blocks(const rb_plan *p, int *blk_m, int *blk_n,

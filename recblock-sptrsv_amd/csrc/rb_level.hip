@@ -721,7 +721,7 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
     // (levels far too wide for one workgroup are not worth the tables, nor the
     // analysis where their rows alone say so)
     auto too_wide = [&](int nsteps) {
-        return np == 1 && level_us(p, nsteps) > 8.0 * chain_us(p);
+        return p->want_schedule == RB_SCHED_AUTO && np == 1 && level_us(p, nsteps) > 8.0 * chain_us(p);
     };
     if (too_wide(m / 64)) return RB_OK;
     Arena tmp(76 * (size_t)m + (1 << 20));

@@ -608,7 +608,10 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     // steps 4-8 run; the upload follows step 8.  It is made for rows of few
     // entries, most of them in the wave's previous step; for longer rows the
     // level schedule is built first, and alone where it is clearly faster.
-    const bool level_first = p->want_schedule == RB_SCHED_AUTO && nnz > 4L * m;
+    const bool chosen = p->want_schedule == RB_SCHED_AUTO;  // by the tuner
+    const bool level_only = p->want_schedule == RB_SCHED_LEVEL,
+               flow_only = p->want_schedule == RB_SCHED_FLOW;
+    const bool level_first = level_only || (chosen && nnz > 4L * m);
     FusedJob *fjob = nullptr;
     struct JobGuard {  // an early return abandons the job (joins the thread)
         FusedJob *&j;
@@ -619,7 +622,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     double fused_ms = 0.0;
     auto start_fused = [&]() -> rb_status {
         auto t = std::chrono::steady_clock::now();
-        if (p->want_schedule != RB_SCHED_BLOCKED && m > 0)
+        if (p->want_schedule != RB_SCHED_BLOCKED && !level_only && !flow_only && m > 0)
             RB_TRY(build_fused_start(p, prptr, ccol, cval, p->fused_waves, s, &fjob));
         fused_ms = std::chrono::duration<double, std::milli>(
                        std::chrono::steady_clock::now() - t)
@@ -876,7 +879,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     auto t_f1 = std::chrono::steady_clock::now();
 
     mark("fused");
-    if (p->want_schedule == RB_SCHED_AUTO && !level_first && m > 0) {
+    if (chosen && !level_first && m > 0) {
         bool narrow = !p->fused;
         if (!narrow) RB_TRY(level_narrow(p, s, &narrow));
         if (narrow) RB_TRY(build_level(p, prptr, ccol, cval, s));
@@ -884,9 +887,14 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     mark("level");
     // flow schedule, for what neither of the others is made for
     // (a mixed plan keeps the fused one, which has an FP32 form)
-    if (p->want_schedule == RB_SCHED_AUTO && (level_first || !p->fused) &&
-        !(p->mixed && p->fused) && !level_beats_walk(p))
+    if (flow_only || (chosen && (level_first || !p->fused) && !(p->mixed && p->fused) &&
+                      !level_beats_walk(p)))
         RB_TRY(build_flow(p, prptr, ccol, cval, s));
+    if (m > 0 && ((level_only && !p->level) || (flow_only && !p->flow))) {
+        set_error(RB_ERR_INVALID_ARG, level_only ? "the factor does not fit the level schedule"
+                                                 : "the factor does not fit the flow schedule");
+        return RB_ERR_INVALID_ARG;
+    }
     mark("flow");
     // ---- 10. FP32 + FP64-refinement storage: FP32 copies of the slot
     // values, and the original matrix as CSR for the FP64 residuals (rows,

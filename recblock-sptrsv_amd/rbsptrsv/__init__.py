@@ -6,6 +6,6 @@ workload generators.
 """
 from . import gen  # noqa: F401
 from ._lib import (EXPORTS, LIB_PATH, RbError, SCHED_AUTO, SCHED_BLOCKED,  # noqa: F401
-                   SCHED_FUSED, build, lib)
+                   SCHED_FLOW, SCHED_FUSED, SCHED_LEVEL, build, lib)
 from .api import (Batch, Plan, lv_auto, recblocking_solver,  # noqa: F401
                   recblocking_solver_cuda, set_bench_repeat)

@@ -28,6 +28,7 @@ EXPORTS = [
     "rb_batch_plan", "rb_batch_destroy",
     "rb_mmio_info", "rb_mmio_data", "rb_mmio_triangle",
     "rb_solve_noalloc", "rb_noalloc_limit", "rb_plan_block_kernels",
+    "rb_plan_schedule",
 ]
 
 RB_OK = 0
@@ -36,7 +37,7 @@ STATUS_NAMES = {0: "RB_OK", 1: "RB_ERR_INVALID_ARG", 2: "RB_ERR_NOT_SQUARE",
                 5: "RB_ERR_ZERO_DIAG", 6: "RB_ERR_HIP", 7: "RB_ERR_NO_MEMORY",
                 8: "RB_ERR_INTERNAL", 9: "RB_ERR_NOT_CONVERGED"}
 
-SCHED_AUTO, SCHED_BLOCKED, SCHED_FUSED = 0, 1, 2
+SCHED_AUTO, SCHED_BLOCKED, SCHED_FUSED, SCHED_LEVEL, SCHED_FLOW = 0, 1, 2, 3, 4
 
 
 class RbError(RuntimeError):
@@ -107,6 +108,8 @@ def lib():
     L.rb_plan_destroy.restype = i
     L.rb_plan_info_get.argtypes = [vp, ctypes.POINTER(rb_plan_info)]
     L.rb_plan_info_get.restype = i
+    L.rb_plan_schedule.argtypes = [vp]
+    L.rb_plan_schedule.restype = i
     L.rb_plan_blocks.argtypes = [vp] + [vp] * 15
     L.rb_plan_blocks.restype = i
     L.rb_plan_block_kernels.argtypes = [vp, vp, vp, vp]

@@ -155,6 +155,10 @@ class Plan:
         check(lib().rb_plan_info_get(self._h, ctypes.byref(inf)))
         return inf
 
+    def schedule(self):
+        """The schedule a solve runs, SCHED_BLOCKED .. SCHED_FLOW."""
+        return lib().rb_plan_schedule(self._h)
+
     # ------------------------------------------------------------ solve
     def solve(self, b, x=None, stream=None):
         """Solve for b: shape (m,) or (m, k), column-major on the device
@@ -337,6 +341,9 @@ class Batch:
         check(lib().rb_plan_info_get(lib().rb_batch_plan(self._h),
                                      ctypes.byref(inf)))
         return inf
+
+    def schedule(self):
+        return lib().rb_plan_schedule(lib().rb_batch_plan(self._h))
 
     def _tables(self, bs, xs):
         torch = _torch()
