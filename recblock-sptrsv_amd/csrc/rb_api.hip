@@ -149,12 +149,14 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     // launches of 4.5 us: not timed where another schedule takes less than
     // half of the one or less than the other (500 x 500 grid, 999 levels, 70
     // us: timing the first block alone took 2.6 ms).  A mixed plan on the flow
-    // schedule refines on the walk.
-    const bool clear = pick >= 0 && !(pick == kFlow && p->mixed) &&
-                       best < std::max(0.45e-3 * p->nlevel, 0.018);
+    // schedule refines on the walk, whose kernels are then all timed (20,000
+    // rows of 200 entries backward, refined: 369 ms with the timing stopped
+    // early, 282 with all of them).
+    const bool walks = pick == kFlow && p->mixed;
+    const bool clear = pick >= 0 && !walks && best < std::max(0.45e-3 * p->nlevel, 0.018);
     if (st == RB_OK)
-        st = tune_blocks(p, clear ? 1 : block_mode, s, k == 1 && pick >= 0 ? 2.0 * best : 0.0,
-                         &cut);
+        st = tune_blocks(p, clear ? 1 : block_mode, s,
+                         k == 1 && pick >= 0 && !walks ? 2.0 * best : 0.0, &cut);
     if (st == RB_OK && !cut && !clear) {
         (void)timed(kBlocked, 1);  // warm (captures the walk)
         const double t1 = timed(kBlocked, 1);
