@@ -611,7 +611,8 @@ __global__ void k_ir_update(const float *__restrict__ d, int m, double *x,
 
 // r = b - A x in the original ordering, FP64, over the original matrix as
 // CSR (rows, b, r and x all in the caller's order); max |r| per column.
-// For matrices whose rows reach too far for the kernel below: G lanes per row
+// For matrices whose rows reach too far or are too long for the kernel below,
+// and for few rows: G lanes per row
 // (a power of two at or above the mean row
 // length, as for the square blocks' SpMV) read the row's entries coalesced
 // and sum them in a fixed order (a thread per row was slow on the
@@ -725,17 +726,24 @@ static void residual_kc(rb_plan *p, int nc, const double *b, long ldb,
 // win[block]: first column and past the last of the block's rows.
 constexpr int kResT = 512, kResPer = 2, kResRows = kResT * kResPer, kResCols = 8;
 constexpr int kResWin = 7680;  // columns of a window at most (60 KB)
+// Longer rows keep a thread on its own behind the registers: 32 columns of
+// 100,000 rows, refined, window / gathers: 17 entries in every row 1,590 / 1,467
+// us, 13 in every row 1,138 / 1,207; 4 in most and 31 in every thousandth 570 /
+// 630, in every 50th 726 / 754; 64 in every 50th 960 / 830.  (3,000 power-law
+// rows, the longest of 512, 8 columns: 1,153 / 581.)
+constexpr int kResLong = 32, kResMean = 14;  // entries: longest row, mean
+constexpr int kResFull = 192, kResLeast = 48;  // workgroups (residual())
 template <int kResEnt>
 __global__ void __launch_bounds__(kResT)
     k_ir_residual_win(const int *__restrict__ rptr, const int *__restrict__ rcol,
                       const double *__restrict__ rval, int m, int ncol,
                       const double *__restrict__ b, long ldb, const double *__restrict__ x,
                       long ldx, double *r, const int2 *__restrict__ win, RowCols cols,
-                      unsigned long long *rmax, const int *__restrict__ done) {
+                      int group, unsigned long long *rmax, const int *__restrict__ done) {
     extern __shared__ double xs[];
     __shared__ unsigned long long lmax[kResCols];
     __shared__ int widest;
-    const int c0 = blockIdx.y * kResCols, c1 = min(ncol, c0 + kResCols);
+    const int c0 = blockIdx.y * group, c1 = min(ncol, c0 + group);
     bool any = false;
     for (int c = c0; c < c1; c++) any = any || !done[c];
     if (!any) return;  // the whole workgroup
@@ -804,38 +812,52 @@ __global__ void __launch_bounds__(kResT)
 
 __global__ void __launch_bounds__(kResT)
     k_ir_window(const int *__restrict__ rptr, const int *__restrict__ rcol, int m, int2 *win,
-                int *most) {
-    __shared__ int lo, hi;
+                int *most, int *longest) {
+    __shared__ int lo, hi, rows;
     if (threadIdx.x == 0) {
         lo = 0x7fffffff;
-        hi = 0;
+        hi = rows = 0;
     }
     __syncthreads();
-    int l = 0x7fffffff, h = 0;
+    int l = 0x7fffffff, h = 0, len = 0;
     for (int k = 0; k < kResPer; k++) {
         const int i = blockIdx.x * kResRows + k * kResT + threadIdx.x;
-        each_entry(i < m ? rptr[i] : 0, i < m ? rptr[i + 1] : 0, [&](int q) {
+        const int a = i < m ? rptr[i] : 0, e = i < m ? rptr[i + 1] : 0;
+        len = max(len, e - a);
+        each_entry(a, e, [&](int q) {
             l = min(l, rcol[q]);
             h = max(h, rcol[q] + 1);
         });
     }
     atomicMin(&lo, l);
     atomicMax(&hi, h);
+    atomicMax(&rows, len);
     __syncthreads();
     if (threadIdx.x == 0) {
         win[blockIdx.x] = make_int2(lo, hi);
         atomicMax(most, hi - lo);
+        atomicMax(longest, rows);
     }
 }
 
 static void residual(rb_plan *p, int nc, const double *b, long ldb,
                      const double *x, long ldx, hipStream_t s) {
-    if (p->rwin > 0) {
+    // The window's workgroups take their columns one after another: up to
+    // kResCols, but no more than leave kResFull workgroups (refined solves of
+    // 8 columns, us, with 8 columns each / this / the gathers: 12,000 banded
+    // rows of 10 entries 224 / 190 / 202, 100,000 rows 940 / 923 / 972).
+    // Fewer than kResLeast leave the chip to latency (one column, the window
+    // against the gathers: 12,000 rows 183 and 174, 25,000 292 and 291,
+    // 102,400 of a grid 169 and 180).
+    const int blocks = nblk(p->m, kResRows);
+    int group = kResCols;
+    while (group > 1 && blocks * ((nc + group - 1) / group) < kResFull) group /= 2;
+    const int wgs = blocks * ((nc + group - 1) / group);
+    if (p->rwin > 0 && wgs >= kResLeast) {
         auto *kern = (long)p->nnz <= 4L * p->m ? k_ir_residual_win<4> : k_ir_residual_win<10>;
-        kern<<<dim3(nblk(p->m, kResRows), (nc + kResCols - 1) / kResCols), kResT,
-               sizeof(double) * p->rwin, s>>>(
+        kern<<<dim3(blocks, wgs / blocks), kResT, sizeof(double) * p->rwin, s>>>(
             p->d_rptr, p->d_rcol, p->d_rval, p->m, nc, b, ldb, x, ldx, p->d_r, p->d_rwin,
-            RowCols{p->d_part, p->d_partcap}, p->d_norms + nc, p->d_irdone);
+            RowCols{p->d_part, p->d_partcap}, group, p->d_norms + nc, p->d_irdone);
         return;
     }
     switch (cols_per_thread(nc)) {
@@ -1388,15 +1410,15 @@ rb_status tune_blocks(rb_plan *p, int mode, hipStream_t s, double budget_ms,
 // the windows of the residual, if they fit (after d_rptr and d_rcol are there)
 rb_status residual_windows(rb_plan *p, Arena &tmp, hipStream_t s) {
     const int nb = nblk(p->m, kResRows);
-    int *most, h = 0;
-    RB_TRY(tmp.alloc(&most, 1));
+    int *most, h[2] = {0, 0};  // widest window, longest row
+    RB_TRY(tmp.alloc(&most, 2));
     RB_TRY(p->arena.alloc(&p->d_rwin, nb));
-    RB_HIP(hipMemsetAsync(most, 0, sizeof(int), s));
-    k_ir_window<<<nb, kResT, 0, s>>>(p->d_rptr, p->d_rcol, p->m, p->d_rwin, most);
+    RB_HIP(hipMemsetAsync(most, 0, sizeof(h), s));
+    k_ir_window<<<nb, kResT, 0, s>>>(p->d_rptr, p->d_rcol, p->m, p->d_rwin, most, most + 1);
     RB_HIP(hipGetLastError());
-    RB_HIP(hipMemcpyAsync(&h, most, sizeof(int), hipMemcpyDeviceToHost, s));
+    RB_HIP(hipMemcpyAsync(h, most, sizeof(h), hipMemcpyDeviceToHost, s));
     RB_HIP(hipStreamSynchronize(s));
-    p->rwin = h <= kResWin ? h : 0;
+    p->rwin = h[0] <= kResWin && h[1] <= kResLong && (long)p->nnz <= (long)kResMean * p->m ? h[0] : 0;
     return RB_OK;
 }
 

@@ -53,3 +53,32 @@ def test_refined_solve_matches_oracle(oracle, name, n, rows_of, reach, lower):
             assert residual(f, X[:, j], B[:, j]) < 1e-12
     p.check()
     p.close()
+
+
+# groups of 1, 2, 4 and 8 columns to a workgroup (so many that at least 192
+# workgroups are left), too few workgroups for it (48), and the longest row it
+# takes and one more
+@pytest.mark.parametrize("n,rows_of,ks", [
+    (3000, [3], (15, 16, 17)),
+    (25000, [3, 9], (1, 2, 7, 8, 9)),
+    (60000, [2], (1, 4, 9, 24)),
+    (200000, [3], (1, 8, 9)),
+    (50000, [3] * 40 + [31], (1, 9)),
+    (50000, [3] * 40 + [32], (1, 9)),
+], ids=lambda v: str(v[-1]) if isinstance(v, list) else str(v).replace(" ", ""))
+def test_residual_groups(oracle, n, rows_of, ks):
+    import torch
+    from rbsptrsv import Plan
+    f = _reach(n, rows_of, 700, seed=n)
+    print("residual groups", n, rows_of[-1], flush=True)
+    rp, ci, v = f.csr()
+    B = gen.rhs(f.n, seed=4, k=max(ks))
+    p = Plan.from_factor(f, mixed=True)
+    for k in ks:
+        b = torch.as_tensor(np.ascontiguousarray(B[:, :k].T), device="cuda")
+        X = p.solve_f32ir(b.t())[0].t().cpu().numpy()
+        for j in range(k):
+            assert residual(f, X[j], B[:, j]) < 1e-12
+        assert rel_err(X[k - 1], oracle.sptrsv_serial(rp, ci, v, f.n, 0, B[:, k - 1])) < 1e-10
+    p.check()
+    p.close()
