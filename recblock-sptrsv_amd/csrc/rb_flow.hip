@@ -25,7 +25,10 @@
 // Several right-hand sides: a row's x lie together, CP columns per lane on
 // CL neighbouring lanes, so that an entry costs one line for all of them
 // (300,001 rows backward, 5 columns: 160 us; column by column, an entry at a
-// time, 1,210 us).
+// time, 1,210 us).  Groups of columns go side by side in one launch, on as
+// many workgroups together as one alone has at most (32 columns of 300,000 rows
+// 527 us; with up to twice as many 783, with that many for each 1,567: the
+// waves beyond only poll).
 //
 // x is divided by the diagonal (a product with its reciprocal is no faster
 // here, and further off: 1.03e-16 of 4M rows, 5.6e-17 like this).
@@ -49,6 +52,8 @@ constexpr int kEnt = 4;      // entries per lane at a time
 constexpr int kWaves = 16;   // waves of a workgroup, each with a ticket counter of its own
 constexpr int kPad = 32;     // counters apart (ints)
 constexpr int kCtl = (kWaves + 1) * kPad;  // and the count of finished workgroups
+constexpr int kCols = 8;     // columns of a row's line of x at most
+constexpr int kGroups = 4;   // lines of that many, a launch
 
 inline int nblk(long n, int t = kT) { return (int)((n + t - 1) / t); }
 
@@ -70,10 +75,11 @@ struct FlowArgs {
     const double *b;
     double *x;
     long ldb, ldx;
-    int ncol;           // columns, at most the kernel's
+    int ncol;           // columns, at most the kernel's times the grid's groups
     int m, nsteps;
-    double *xs;         // [m][columns of the kernel] x by position, the sentinel until solved
-    int *ctl;           // [kCtl] tickets; workgroups done
+    double *xs;         // [groups][m][columns of the kernel] x by position, the
+                        // sentinel until solved
+    int *ctl;           // [groups][kCtl] tickets; workgroups done
     int *status;
     unsigned spin;
 };
@@ -111,26 +117,33 @@ __device__ inline void st_x(Xv<CP> v, __amdgpu_buffer_rsrc_t r, int off) {
         __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, off, 0, kSC1);
 }
 
-__global__ void __launch_bounds__(kT) k_flow_reset(double *xs, long n, int *ctl) {
+__global__ void __launch_bounds__(kT) k_flow_reset(double *xs, long n, int *ctl, int nctl) {
     const long i = ((long)blockIdx.x * kT + threadIdx.x) * 2;
     const double s = __longlong_as_double((long long)kPending);
     if (i + 1 < n) *(double2 *)(xs + i) = make_double2(s, s);
     else if (i < n) xs[i] = s;
     if (blockIdx.x == 0)
-        for (int k = threadIdx.x; k < kCtl; k += kT) ctl[k] = 0;
+        for (int k = threadIdx.x; k < nctl; k += kT) ctl[k] = 0;
 }
 
 // CP columns per lane, CL lanes beside each other for a row's columns: an
 // entry's CP * CL columns of x lie together and are read by CL lanes in one
-// access.  A wave takes 64 / CL of a step's 64 lanes at a time.
-template <int CP, int CL>
+// access.  A wave takes 64 / CL of a step's 64 lanes at a time.  MULTI:
+// blockIdx.y is a group of CP * CL columns, with tickets and x of its own, which
+// waits for no other.  (The one group of the others is known to be the first:
+// 5 columns of 300,001 rows 194 us, 196 with the multiple form.)
+template <int CP, int CL, bool MULTI>
 __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
     constexpr int KC = CP * CL, S = 64 / CL;
+    const int grp = MULTI ? blockIdx.y : 0, g0 = grp * KC;
+    const int ncol = a.ncol - g0;  // the group's columns
+    const double *b = a.b + g0 * a.ldb;
+    double *xo = a.x + g0 * a.ldx;
     const int lane = threadIdx.x & 63, c0 = lane % CL * CP;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const __amdgpu_buffer_rsrc_t xs = __builtin_amdgcn_make_buffer_rsrc(
-        a.xs, (short)0, (int)min((long)a.m * KC * 8, 0x7fffffffL), 0x00020000);
-    int *ticket = a.ctl + wave * kPad;
+        a.xs + (long)g0 * a.m, (short)0, (int)min((long)a.m * KC * 8, 0x7fffffffL), 0x00020000);
+    int *ticket = a.ctl + grp * kCtl + wave * kPad;
     auto take = [&]() {
         int t = 0;
         if (lane == 0)
@@ -206,7 +219,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
         };
 #pragma unroll
         for (int c = 0; c < CP; c++)
-            bv[c] = live && c0 + c < a.ncol ? a.b[(c0 + c) * a.ldb + row] : 0.0;
+            bv[c] = live && c0 + c < ncol ? b[(c0 + c) * a.ldb + row] : 0.0;
         auto tree = [&](int rep, double (&sum)[CP]) {
 #pragma unroll
             for (int c = 0; c < CP; c++) acc[c] = 0.0;
@@ -235,7 +248,7 @@ __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
             st_x<CP>(x, xs, (p * KC + c0) * 8);
 #pragma unroll
             for (int c = 0; c < CP; c++)
-                if (c0 + c < a.ncol) a.x[(c0 + c) * a.ldx + row] = x.v[c];
+                if (c0 + c < ncol) xo[(c0 + c) * a.ldx + row] = x.v[c];
         }
     }
     // the last workgroup turns every x into a NaN when a wait gave up
@@ -243,7 +256,8 @@ __global__ void __launch_bounds__(kWaves * 64) k_flow(FlowArgs a) {
     __shared__ int last;
     if (threadIdx.x == 0)
         last = __hip_atomic_fetch_add(a.ctl + kWaves * kPad, 1, __ATOMIC_ACQ_REL,
-                                      __HIP_MEMORY_SCOPE_AGENT) == (int)gridDim.x - 1 &&
+                                      __HIP_MEMORY_SCOPE_AGENT) ==
+                   (int)(gridDim.x * (MULTI ? gridDim.y : 1)) - 1 &&
                (__hip_atomic_load(a.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & 7);
     __syncthreads();
     if (last)
@@ -430,7 +444,7 @@ rb_status build_flow(rb_plan *p, const int *d_rp, const int *d_cc, const double 
     RB_TRY(A.alloc(&F->d_val, ne));
     RB_TRY(A.alloc(&F->d_row, m));
     RB_TRY(A.alloc(&F->d_diag, m));
-    RB_TRY(A.alloc(&F->d_ctl, 2 * kCtl));
+    RB_TRY(A.alloc(&F->d_ctl, 2 * kGroups * kCtl));
     k_fl_blank<<<nblk((long)ne), kT, 0, s>>>(F->d_col, F->d_val, (long)ne);
     k_fl_fill<<<nblk(m), kT, 0, s>>>(key, run, rend, order, head, sidx, off, g, d_rp, d_cc, d_cv,
                                      newpos, p->d_levelItem, F->d_step, F->d_col, F->d_val,
@@ -449,40 +463,53 @@ template <int CP, int CL>
 static rb_status flow_columns(rb_plan *p, const double *b, long ldb, double *x, long ldx,
                               int ncol, double *xs, int *ctl, hipStream_t s) {
     const FlowPlan *F = p->flow;
-    const long n = (long)p->m * CP * CL;
-    k_flow_reset<<<nblk((n + 1) / 2), kT, 0, s>>>(xs, n, ctl);
+    const int groups = (ncol + CP * CL - 1) / (CP * CL);
+    const long n = (long)p->m * CP * CL * groups;
+    k_flow_reset<<<nblk((n + 1) / 2), kT, 0, s>>>(xs, n, ctl, groups * kCtl);
     FlowArgs a{F->d_step, F->d_col, F->d_val, F->d_row, F->d_diag, b, x, ldb, ldx, ncol,
                p->m, F->nsteps, xs, ctl, p->d_status, p->spin_limit};
     const long takes = (long)F->nsteps * CL;
     const int grid = (int)std::max(
         std::min(16L, (takes + kWaves - 1) / kWaves),
-        std::min((long)F->ncu, 10 * takes / ((long)kWaves * std::max(1, p->nlevel))));
+        std::min((long)F->ncu / groups, 10 * takes / ((long)kWaves * std::max(1, p->nlevel))));
     mark_start(p, s);
-    k_flow<CP, CL><<<grid, kWaves * 64, 0, s>>>(a);
+    if (groups > 1)
+        k_flow<2, kCols / 2, true><<<dim3(grid, groups), kWaves * 64, 0, s>>>(a);
+    else
+        k_flow<CP, CL, false><<<grid, kWaves * 64, 0, s>>>(a);
     RB_HIP(hipGetLastError());
     mark_end(p, s);
     return RB_OK;
 }
 
-// the x buffer of n columns together: m values each for 1, 2, 4 or 8
-static int flow_width(int n) { return n <= 2 ? n : n <= 4 ? 4 : 8; }
+// the x buffer of n columns together: m values each for 1, 2, 4 or 8, or for
+// groups of 8
+static int flow_width(int n) {
+    return n <= 2 ? n : n <= 4 ? 4 : (n + kCols - 1) / kCols * kCols;
+}
 
 rb_status solve_flow(rb_plan *p, const double *d_b, int ldb, double *d_x, int ldx, int nrhs,
                      hipStream_t s, double *ws, size_t ws_bytes) {
     const int m = p->m;
     if (m == 0) return RB_OK;
     const size_t col = sizeof(double) * (size_t)m;
-    int cap = 8;  // columns at a time
+    // columns at a time: a power of two up to a group, or whole groups (one
+    // after another each pays the chain of levels: 32 columns of 30,000
+    // power-law rows 646 us, of 900,000 2,119; together 175 and 1,642; the
+    // block walk 416 and 3,274)
+    int cap = kCols;
     while (cap > 1 && (long)m * cap * 8 > 0x7fffffffL) cap /= 2;
+    if (cap == kCols) cap = std::max(1, std::min(kGroups, walk_cols(p) / kCols)) * kCols;
     // a group's b is copied first where x would overwrite what is still to be
     // read
     const bool copy = part_overlap(d_b, ldb, d_x, ldx, m, nrhs);
     int group = copy ? std::min(nrhs, walk_cols(p)) : nrhs;  // columns copied at a time
     double *xs = ws, *bc = nullptr;
     // (a solve on a caller's workspace may run beside one on the plan's)
-    int *ctl = p->flow->d_ctl + (ws ? kCtl : 0);
+    int *ctl = p->flow->d_ctl + (ws ? kGroups * kCtl : 0);
     if (ws) {
         if (copy) group = 1;
+        while (cap > kCols && cap * col > ws_bytes) cap -= kCols;
         while (cap > 1 && cap * col > ws_bytes) cap /= 2;
         if ((copy ? 2 : 1) * col > ws_bytes) {
             set_error(RB_ERR_INVALID_ARG, "workspace too small for one column");

@@ -67,6 +67,13 @@ def test_flow(oracle, torch, name, make, lower):
     _matches_oracle(oracle, torch, f, SCHED_FLOW, [2, 3, 4, 5, 8, 9])
 
 
+@pytest.mark.parametrize("n", [20001, 60000])
+def test_flow_groups(oracle, torch, n):
+    """Groups of 8 columns side by side in a launch, up to four of them."""
+    _matches_oracle(oracle, torch, gen.powerlaw(n, seed=5), SCHED_FLOW,
+                    [7, 15, 16, 17, 24, 25, 31, 32, 33, 40])
+
+
 def test_level_special_values(oracle, torch):
     """An infinite and a NaN right-hand side entry spread to the rows that
     depend on them and to no other."""
@@ -83,7 +90,7 @@ def test_level_special_values(oracle, torch):
     assert rel_err(x[fine], xo[fine]) < 1e-10
 
 
-@pytest.mark.parametrize("k", [1, 3])
+@pytest.mark.parametrize("k", [1, 3, 19])
 @pytest.mark.parametrize("name,make,schedule", [
     ("flow", lambda: gen.powerlaw(60000, seed=5), SCHED_FLOW),
     # (several waves, so that one has to wait for another)
