@@ -155,7 +155,7 @@ static rb_status choose_schedule(rb_plan *p, int block_mode, hipStream_t s) {
     const bool walks = pick == kFlow && p->mixed;
     const bool clear = pick >= 0 && !walks && best < std::max(0.45e-3 * p->nlevel, 0.018);
     if (st == RB_OK)
-        st = tune_blocks(p, clear ? 1 : block_mode, s,
+        st = tune_blocks(p, clear && block_mode == 0 ? 1 : block_mode, s,
                          k == 1 && pick >= 0 && !walks ? 2.0 * best : 0.0, &cut);
     if (st == RB_OK && !cut && !clear) {
         (void)timed(kBlocked, 1);  // warm (captures the walk)
