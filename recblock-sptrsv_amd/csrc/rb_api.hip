@@ -453,7 +453,7 @@ rb_status rb_plan_info_get(const rb_plan *p, rb_plan_info *info) {
     info->nlevel = p->nlevel;
     info->schedule = p->schedule;
     info->preprocess_ms = p->preprocess_ms;
-    info->device_bytes = p->arena.bytes + level_bytes(p) + flow_bytes(p);
+    info->device_bytes = p->arena.bytes + fused_bytes(p) + level_bytes(p) + flow_bytes(p);
     for (int i = 0; i < 4; i++) info->phase_ms[i] = p->phase_ms[i];
     info->tune_ms[0] = p->tune_ms_blocked;
     info->tune_ms[1] = p->tune_ms_fused;

@@ -1115,6 +1115,7 @@ __global__ void __launch_bounds__(kTileThreads)
 
 struct FusedPlan {
     int W = 0, NDPP = 0, NRING = 0, K = 0, nsteps = 0, nent = 0, npub = 0;
+    Arena mem;  // the tables below
     bool blk = false;  // FIFO checked once per block (wait graph acyclic)
     unsigned epoch = 0;  // solves run; selects the slot-order x buffer
     int *d_step0 = nullptr, *d_gent0 = nullptr, *d_pub0 = nullptr;
@@ -1658,7 +1659,7 @@ rb_status build_fused_host(rb_plan *p, const HostVec<int> &rp,
     F->nsteps = NS;
     F->nent = gent0[W];
     F->npub = pub0[W];
-    Arena &A = p->arena;
+    Arena &A = F->mem;
     const size_t nslots = (size_t)NS * 64;
     RB_TRY(A.alloc(&F->d_step0, W + 1));
     RB_TRY(A.alloc(&F->d_gent0, W + 1));
@@ -1888,7 +1889,10 @@ FusedPlan::~FusedPlan() {
     for (void *q : {(void *)d_xq, (void *)d_brec, (void *)d_gval32,
                     (void *)d_tinvd32, (void *)d_xq32, (void *)d_brec32})
         if (q) (void)hipFree(q);
+    mem.release();
 }
+
+size_t fused_bytes(const rb_plan *p) { return p->fused ? p->fused->mem.bytes : 0; }
 
 // other plans whose launches may be resident beside this one's
 static int others(const FusedPlan *F) {

@@ -370,6 +370,7 @@ rb_status solve_flow(rb_plan *p, const double *d_b, int ldb, double *d_x, int ld
 void flow_destroy(rb_plan *p);
 size_t flow_bytes(const rb_plan *p);
 size_t level_bytes(const rb_plan *p);
+size_t fused_bytes(const rb_plan *p);
 // the same solves on caller-provided per-solve buffers (ws, ws_bytes)
 // instead of the plan's: the blocked walk needs blocked_ws_bytes(p) (one
 // column at a time, eager launches), the fused schedule 16 bytes per slot

@@ -2,7 +2,7 @@
 import numpy as np
 import pytest
 
-from rbsptrsv import SCHED_AUTO, SCHED_BLOCKED, SCHED_FLOW, gen
+from rbsptrsv import SCHED_AUTO, SCHED_BLOCKED, SCHED_FLOW, SCHED_LEVEL, gen
 
 pytestmark = pytest.mark.gpu
 
@@ -37,3 +37,18 @@ def test_block_kernels_asked_for_are_kept(mode, kern):
         p.close()
     assert kern in got[1]
     assert np.array_equal(*got)
+
+
+def test_losing_schedules_leave_nothing():
+    """A plan holds the tables of the schedule it runs, as if asked for by
+    name, not those of the others that were built and timed."""
+    from rbsptrsv import Plan
+    f = gen.banded(20000, seed=4).transpose()
+    held = []
+    for schedule in (SCHED_AUTO, SCHED_LEVEL):
+        # (for many columns the fused schedule is built besides)
+        p = Plan.from_factor(f, schedule=schedule, tune_rhs=32)
+        assert p.schedule() == SCHED_LEVEL
+        held.append(p.info().device_bytes)
+        p.close()
+    assert held[0] == held[1]
