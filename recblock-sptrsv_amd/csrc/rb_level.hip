@@ -444,12 +444,23 @@ __global__ void k_lv_need(int m, const int *__restrict__ rp, const int *__restri
         r, live ? level[r] : 0);
 }
 
+// Blocks of kBlock rows, counted part by part (a part's rows lie together; its
+// first row and block: off and blk0, null for a single part)
+struct RowBlocks {
+    const int *part, *off, *blk0;
+    __device__ int part_of(int row) const { return part ? part[row] : 0; }
+    __device__ int of(int row) const {
+        const int p = part_of(row);
+        return (off ? blk0[p] : 0) + (row - (off ? off[p] : 0)) / kBlock;
+    }
+};
+
 __global__ void k_lv_block_start(int m, const int *__restrict__ level,
                                  const int *__restrict__ need, const int *__restrict__ lf,
-                                 int *start) {
+                                 RowBlocks rb, int *start) {
     const int r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= m || need[r] == 0x7fffffff) return;
-    int *at = start + lf[r] / kBlock;
+    int *at = start + rb.of(lf[r]);
     const int l = max(level[r], need[r] - kAhead);
     if (*(volatile int *)at > l) atomicMin(at, l);
 }
@@ -457,15 +468,14 @@ __global__ void k_lv_block_start(int m, const int *__restrict__ level,
 // solve-order row q: its sort key (part, level, log2 lanes per row)
 __global__ void k_lv_key(RowGeom g, const int *__restrict__ rp, const int *__restrict__ level,
                          const int *__restrict__ need, const int *__restrict__ start,
-                         const int *__restrict__ lf, const int *__restrict__ part, int *key,
-                         int *val) {
+                         const int *__restrict__ lf, RowBlocks rb, int *key, int *val) {
     const int q = blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.m) return;
     const int r = g.fwd ? q : g.m - 1 - q;
-    const int len = rp[r + 1] - rp[r] - 1, p = part ? part[lf[r]] : 0;
+    const int len = rp[r + 1] - rp[r] - 1, p = rb.part_of(lf[r]);
     int l = max(level[r], need[r] - kAhead);
     if (need[r] == 0x7fffffff) {
-        const int s = start[lf[r] / kBlock];
+        const int s = start[rb.of(lf[r])];
         l = s == 0x7fffffff ? level[r] : max(level[r], s);
     }
     key[q] = (p * g.nlev + l) * 8 + glog_of(min(len, kMaxLen));
@@ -738,22 +748,6 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
     const RowGeom g{m, p->subst == 0, p->nlevel};
     RB_HIP(hipMemsetAsync(cnt, 0, sizeof(int), s));
     RB_HIP(hipMemsetAsync(head + m, 0, sizeof(int), s));
-    // (run, lev, newpos and rend are free until the rows are sorted)
-    k_lv_own<<<nblk(m), kT, 0, s>>>(g, d_rp, p->d_levelPtr, lev, newpos, cnt);
-    k_lv_need<<<nblk(m), kT, 0, s>>>(m, d_rp, d_cc, lev, newpos);
-    k_lv_set<<<nblk(nblk(m, kBlock)), kT, 0, s>>>(rend, nblk(m, kBlock), 0x7fffffff);
-    k_lv_block_start<<<nblk(m), kT, 0, s>>>(m, lev, newpos, p->d_levelItem, rend);
-    k_lv_key<<<nblk(m), kT, 0, s>>>(g, d_rp, lev, newpos, rend, p->d_levelItem, p->d_part, k0,
-                                    v0);
-    RB_HIP(hipGetLastError());
-    RB_TRY(sort_pairs_i32(k0, key, v0, order, m, bits_for((long)np * p->nlevel * 8), s, tmp));
-    k_lv_heads<<<nblk(m), kT, 0, s>>>(key, m, k0, v0);
-    RB_HIP(hipGetLastError());
-    RB_TRY(inclusive_max_i32(k0, run, m, s, tmp));
-    RB_TRY(inclusive_max_i32(v0, lev, m, s, tmp));
-    k_lv_steps<<<nblk(m), kT, 0, s>>>(key, run, lev, order, g, head, rend, newpos);
-    RB_HIP(hipGetLastError());
-    RB_TRY(exclusive_scan_i32(head, sidx, m + 1, s, tmp));
     // the parts' rows and blocks
     std::vector<Part> parts(np);
     std::vector<int> blk0(np + 1, 0);
@@ -764,10 +758,27 @@ rb_status build_level(rb_plan *p, const int *d_rp, const int *d_cc, const double
         blk0[q + 1] = blk0[q] + (parts[q].rows + kBlock - 1) / kBlock;
     }
     const int nb = blk0[np];
-    int *d_blk0, *blk;
+    int *d_blk0, *blk, *start;
     RB_TRY(tmp.alloc(&d_blk0, np));
     RB_TRY(tmp.alloc(&blk, 4 * (size_t)nb));
+    RB_TRY(tmp.alloc(&start, nb));
     RB_HIP(hipMemcpyAsync(d_blk0, blk0.data(), sizeof(int) * np, hipMemcpyHostToDevice, s));
+    const RowBlocks rb{p->d_part, p->d_partoff, d_blk0};
+    // (run, lev and newpos are free until the rows are sorted)
+    k_lv_own<<<nblk(m), kT, 0, s>>>(g, d_rp, p->d_levelPtr, lev, newpos, cnt);
+    k_lv_need<<<nblk(m), kT, 0, s>>>(m, d_rp, d_cc, lev, newpos);
+    k_lv_set<<<nblk(nb), kT, 0, s>>>(start, nb, 0x7fffffff);
+    k_lv_block_start<<<nblk(m), kT, 0, s>>>(m, lev, newpos, p->d_levelItem, rb, start);
+    k_lv_key<<<nblk(m), kT, 0, s>>>(g, d_rp, lev, newpos, start, p->d_levelItem, rb, k0, v0);
+    RB_HIP(hipGetLastError());
+    RB_TRY(sort_pairs_i32(k0, key, v0, order, m, bits_for((long)np * p->nlevel * 8), s, tmp));
+    k_lv_heads<<<nblk(m), kT, 0, s>>>(key, m, k0, v0);
+    RB_HIP(hipGetLastError());
+    RB_TRY(inclusive_max_i32(k0, run, m, s, tmp));
+    RB_TRY(inclusive_max_i32(v0, lev, m, s, tmp));
+    k_lv_steps<<<nblk(m), kT, 0, s>>>(key, run, lev, order, g, head, rend, newpos);
+    RB_HIP(hipGetLastError());
+    RB_TRY(exclusive_scan_i32(head, sidx, m + 1, s, tmp));
     k_lv_set<<<nblk(2 * nb), kT, 0, s>>>(blk, 2 * nb, 0x7fffffff);
     k_lv_set<<<nblk(2 * nb), kT, 0, s>>>(blk + 2 * nb, 2 * nb, 0);
     k_lv_blocks<<<nblk(m), kT, 0, s>>>(key, order, g, d_rp, d_cc, newpos, p->d_levelItem,

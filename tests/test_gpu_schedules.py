@@ -170,3 +170,30 @@ def test_not_for_batches(torch):
     for f, b, x in zip(facs, bs, bt.solve(bs)):
         assert residual(f, x.cpu().numpy(), b.cpu().numpy()) < 1e-12
     bt.close()
+
+
+def test_batch_factors_do_not_move_each_others_rows(torch):
+    """Rows that no other reads, at the head of a factor behind the odd tail of
+    a much deeper one: they keep to their own factor's levels, so that the
+    batch still fits its rings in the caller's order and needs no union columns
+    (2 x 80,100 rows x 16 columns, 20 MB)."""
+    from rbsptrsv import Batch
+    head, tail = 200, gen.banded(19800, seed=3, window=600)
+    cp, ri, v = tail.colptr.astype(np.int64), tail.rowidx, tail.val
+    second = gen.Factor(
+        head + tail.n, np.concatenate([np.arange(head), head + cp]).astype(np.int32),
+        np.concatenate([np.arange(head), head + ri]).astype(np.int32),
+        np.concatenate([np.full(head, 2.0), v]), True)
+    facs = [gen.banded(60100, seed=2), second]
+    bt = Batch(facs, schedule=SCHED_LEVEL)
+    rng = np.random.default_rng(1)
+    bs = [torch.as_tensor(rng.uniform(-1, 1, (16, f.n)), device="cuda").t() for f in facs]
+    xs = [torch.empty_like(b.t()).t() for b in bs]
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    bt.solve(bs, xs=xs)
+    torch.cuda.synchronize()
+    assert free - torch.cuda.mem_get_info()[0] < 10 << 20
+    for f, b, x in zip(facs, bs, xs):
+        assert residual(f, x[:, 0].cpu().numpy(), b[:, 0].cpu().numpy()) < 1e-12
+    bt.close()
