@@ -612,6 +612,12 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     const bool level_only = p->want_schedule == RB_SCHED_LEVEL,
                flow_only = p->want_schedule == RB_SCHED_FLOW;
     const bool level_first = level_only || (chosen && nnz > 4L * m);
+    // (the tuner does without a schedule that no memory is left for)
+    auto if_it_fits = [&](rb_status st) {
+        if (!chosen || st != RB_ERR_NO_MEMORY) return st;
+        set_error(RB_OK, "");
+        return RB_OK;
+    };
     FusedJob *fjob = nullptr;
     struct JobGuard {  // an early return abandons the job (joins the thread)
         FusedJob *&j;
@@ -678,7 +684,7 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     RB_HIP(hipGetLastError());
 
     if (level_first) {
-        RB_TRY(build_level(p, prptr, ccol, cval, s));
+        RB_TRY(if_it_fits(build_level(p, prptr, ccol, cval, s)));
         if (!level_beats_chain(p)) RB_TRY(start_fused());
     }
     mark("slots");
@@ -882,14 +888,14 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     if (chosen && !level_first && m > 0) {
         bool narrow = !p->fused;
         if (!narrow) RB_TRY(level_narrow(p, s, &narrow));
-        if (narrow) RB_TRY(build_level(p, prptr, ccol, cval, s));
+        if (narrow) RB_TRY(if_it_fits(build_level(p, prptr, ccol, cval, s)));
     }
     mark("level");
     // flow schedule, for what neither of the others is made for
     // (a mixed plan keeps the fused one, which has an FP32 form)
     if (flow_only || (chosen && (level_first || !p->fused) && !(p->mixed && p->fused) &&
                       !level_beats_walk(p)))
-        RB_TRY(build_flow(p, prptr, ccol, cval, s));
+        RB_TRY(if_it_fits(build_flow(p, prptr, ccol, cval, s)));
     if (m > 0 && ((level_only && !p->level) || (flow_only && !p->flow))) {
         set_error(RB_ERR_INVALID_ARG, level_only ? "the factor does not fit the level schedule"
                                                  : "the factor does not fit the flow schedule");
