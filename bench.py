@@ -30,8 +30,9 @@ TRAFFIC_FILE = os.path.join(REPO, "profiles", "traffic.json")
 def measured_traffic(workload, schedule):
     """HBM bytes per launch of the dominant kernel from the committed
     rocprofv3 counter runs (FETCH_SIZE + WRITE_SIZE, each scaled by the
-    same counter's reading for a copy kernel of known size), or None when
-    no run covers this workload and schedule."""
+    same counter's reading for a copy kernel of known size) and the kernel
+    that was counted, as the run's entry, or None when none covers this
+    workload and schedule."""
     try:
         with open(TRAFFIC_FILE) as fh:
             tab = json.load(fh)
@@ -40,7 +41,12 @@ def measured_traffic(workload, schedule):
     e = tab.get(workload)
     if not e or e.get("schedule") != schedule:
         return None
-    return e.get("bytes_per_launch")
+    return e
+
+
+SCHEDULES = {1: "blocked", 2: "fused", 3: "level", 4: "flow"}
+KERNELS = {"blocked": "blocked block walk (graph of block kernels)",
+           "fused": "k_staged or k_fused", "level": "k_level", "flow": "k_flow"}
 
 
 def algorithmic_bytes(m, nnz, nrhs=1):
@@ -117,7 +123,8 @@ def f32ir_leg(args, dcp, dri, dv, f, db, K, fp64_ms):
     torch.cuda.synchronize()
     ms = (time.perf_counter() - t0) * 1e3 / args.steps
     q.check()
-    sched = {1: "blocked", 2: "fused"}.get(q.info().schedule, q.info().schedule)
+    # (a plan on the flow schedule refines on the block walk)
+    sched = SCHEDULES[q.schedule()].replace("flow", "blocked")
     q.close()
     X = x.t().cpu().numpy() if K > 1 else x.cpu().numpy()[None, :]
     B = db.t().cpu().numpy() if K > 1 else db.cpu().numpy()[None, :]
@@ -220,7 +227,7 @@ def bench_batch(args):
     t0 = time.perf_counter()
     bt = Batch(facs, lv=-1, schedule=args.schedule, tune_rhs=max(nrhs))
     pre_ms = (time.perf_counter() - t0) * 1e3
-    info = bt.info()
+    info, sched = bt.info(), SCHEDULES[bt.schedule()]
     say("union plan built: %.0f ms, schedule %d (warm solve ms: blocked "
         "%.3f, fused %.3f)" % (pre_ms, info.schedule, info.tune_ms[0],
                                info.tune_ms[1]))
@@ -269,7 +276,7 @@ def bench_batch(args):
                    "factors": len(facs), "rhs_total": K,
                    "n_total": int(sum(f.n for f in facs)),
                    "nnz_total": int(sum(f.nnz for f in facs)),
-                   "schedule": {1: "blocked", 2: "fused"}.get(info.schedule),
+                   "schedule": sched,
                    "levels": info.nlevel, "preprocess_ms": round(pre_ms, 1),
                    "tune_ms": [round(info.tune_ms[0], 3),
                                round(info.tune_ms[1], 3)],
@@ -513,7 +520,10 @@ def main():
 
     B = algorithmic_bytes(f.n, f.nnz, K)
     gbs = B / (ms * 1e-3) / 1e9
-    sched = {1: "blocked", 2: "fused"}.get(info.schedule, info.schedule)
+    sched = SCHEDULES[plan.schedule()]
+    # counter runs cover one right-hand side on the waves the library takes
+    counted = measured_traffic(wname, sched) \
+        if args.rhs == 1 and args.fused_waves == 0 else None
     kern_gbs = B / (launch_ms * 1e-3) / 1e9
     out = {
         "metric": METRIC,
@@ -537,13 +547,8 @@ def main():
         "roofline": {"bound": "hbm", "achieved": round(kern_gbs, 3),
                      "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(kern_gbs / HBM_PEAK_GBS, 5),
-                     # counter runs cover one right-hand side
-                     "traffic": measured_traffic(wname, sched)
-                                if args.rhs == 1 else None,
-                     "kernel": "blocked block walk (graph of block kernels)"
-                               if sched != "fused" else
-                               "k_level or k_flow" if plan.trace() is None
-                               else "k_staged or k_fused",
+                     "traffic": counted and counted["bytes_per_launch"],
+                     "kernel": counted["kernel"] if counted else KERNELS[sched],
                      "launch_ms": round(launch_ms, 5),
                      "algorithmic_bytes_per_launch": B,
                      "cache": "warm: repeated solves, the factor's data "

@@ -293,8 +293,8 @@ rb_status rb::plan_create(const int *d_colptr, const int *d_rowidx, const double
         (void)hipStreamSynchronize((hipStream_t)stream);
         destroy_graph(p);
         fused_destroy(p);
-    level_destroy(p);
-    flow_destroy(p);
+        level_destroy(p);
+        flow_destroy(p);
         p->arena.release();
         delete p;
         return st;

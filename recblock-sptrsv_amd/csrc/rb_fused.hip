@@ -735,11 +735,16 @@ __global__ void __launch_bounds__(kWG)
 // where every workgroup has a compute unit to itself: four more waves stage
 // records and b/diag in LDS, kQ steps of them, and the resolver takes its
 // sums off the staged b/diag.  The consumer is left with two LDS reads, two
-// DPP moves, two FMAs and a store per step, and never waits for memory.
+// DPP moves, two FMAs and a store per step, and waits once a block, for the
+// stagers' loads and the resolver.
 // Bound: issue of one wave (3,000 x 64, one wave: 42 ns a step in k_fused, of
 // which the loads of b and records 4 and 5, clearing the FIFO 4, waiting for
-// memory 9; 30 here) and the hand-offs, 2.6 us each.  (Reading the next block's
-// first steps before its turn: 32 ns; 6 steps ahead instead of 4: alike.)
+// memory 9; 30 here) and the hand-offs from wave to wave.  1500^2, by the
+// trace's counters: the first of 24 waves takes 53 us, 28.6 ns a step and 8 of
+// waits, each later one ends 6.3 after the one before, 1.8 of which are the 64
+// steps between them; with the tables outside the caches 63 and 7.6.  Sixteen
+// columns of 1000^2 on all compute units: 62, then 7.6.  (Reading the next
+// block's first steps before its turn: 32 ns; 6 steps ahead instead of 4: alike.)
 constexpr int kStagers = 4;
 constexpr int kStagedWG = (2 + kStagers) * 64;
 

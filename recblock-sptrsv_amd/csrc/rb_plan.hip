@@ -602,7 +602,6 @@ rb_status build_plan(rb_plan *p, const int *d_colptr, const int *d_rowidx,
     RB_HIP(hipGetLastError());
     RB_TRY(exclusive_scan_i32(prowcnt, prptr, m + 1, s, tmp));
 
-    mark("csr");
     // ---- 9, begun here: the fused schedule's host passes need only the
     // permuted CSR structure and the levels, so they run on a thread while
     // steps 4-8 run; the upload follows step 8.  It is made for rows of few

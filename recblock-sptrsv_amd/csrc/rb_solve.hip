@@ -568,9 +568,10 @@ __device__ inline void raise_max(unsigned long long *at, unsigned long long v) {
     if (__hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < v) atomicMax(at, v);
 }
 
-// max |b| of column blockIdx.y, folded per workgroup.  The first correction reads b itself and writes x (x = 0
-// and r = b as a pass of their own: 212 us of a batch of 1.3M rows x 32
-// columns, 17 us of 880,000 rows; the maxima alone 38 and 7).
+// max |b| of column blockIdx.y, folded per workgroup.  The first correction
+// reads b itself and writes x (x = 0 and r = b as a pass of their own: 212 us of
+// a batch of 1.3M rows x 32 columns, 17 us of 880,000 rows; the maxima alone 38
+// and 7).
 __global__ void __launch_bounds__(kT)
     k_ir_norm(const double *__restrict__ b, long ldb, int m, RowCols cols,
               unsigned long long *bmax) {
@@ -721,8 +722,9 @@ static void residual_kc(rb_plan *p, int nc, const double *b, long ldb,
 // thread keeps the entries of its kResPer rows in registers over the columns
 // of its group (the first kResEnt of a row, 4 or 10 by the mean; what is
 // longer is read again), the window's places two to a word.  Four rows to a
-// thread spilled (with ten entries 249 us), 256 threads were slower (167).  Bound: the bytes of b, r and x (the windows of
-// neighbouring blocks overlap) and the LDS reads, one per entry and column.
+// thread spilled (with ten entries 249 us), 256 threads were slower (167).
+// Bound: the bytes of b, r and x (the windows of neighbouring blocks overlap)
+// and the LDS reads, one per entry and column.
 // win[block]: first column and past the last of the block's rows.
 constexpr int kResT = 512, kResPer = 2, kResRows = kResT * kResPer, kResCols = 8;
 constexpr int kResWin = 7680;  // columns of a window at most (60 KB)
